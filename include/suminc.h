@@ -204,8 +204,10 @@ int suminc_copy_from_device(suminc_ctx* ctx, void* host_dst, const void* dev_src
 int suminc_pr_init(suminc_ctx* ctx);
 /* Runs delta-PageRank rounds until sum|delta| < T or max_rounds: replaces
  * tjn::g_function_pr + tjn::deltaSum (sum_sync_iter_worker.h:885-893, 1372;
- * cudaCode/my_worker.cu:124-142, 304-328).  Returns SUMINC_E_NOT_CONVERGED if the
- * cap is hit (state stays valid). */
+ * cudaCode/my_worker.cu:124-142, 304-328).  A run may take extrapolation steps
+ * (rank += y, delta -= (I - d P^T) y with y a multiple of delta), so it takes fewer
+ * rounds than a loop over suminc_pr_step, to the same stop rule on sum|delta|.
+ * Returns SUMINC_E_NOT_CONVERGED if the cap is hit (state stays valid). */
 int suminc_pr_run(suminc_ctx* ctx, suminc_stats* stats);
 /* One round; residual_out = FP64 sum|delta| before the round. */
 int suminc_pr_step(suminc_ctx* ctx, double* residual_out);

@@ -90,6 +90,15 @@ struct BinLayout {
   uint64_t first = 0, m = 0;  // the value stream's edges: [first, m)
 };
 
+// Extrapolation state of a delta series (extrap.hpp), zero when a run starts.
+struct Extrap {
+  double last;   // the residual of the previous round as chosen
+  double ratio;  // S2 / S1 of the previous round's candidate (0: none)
+  double cand;   // the coefficient the next count evaluates (0: none)
+  double beta;   // the coefficient the state's next vertex pass applies (0: none)
+  double steps;  // extrapolations taken
+};
+
 // Device-side counters block (one allocation, read back in one copy).
 struct Counters {
   unsigned long long wl_count[2];   // worklist lengths (double-buffered frontiers)
@@ -111,6 +120,7 @@ struct Counters {
   unsigned long long hc[3];         // round-indexed heavy-chunk counts
   unsigned long long bcopy[4];      // a batch's group counts, copied out with the counters
   unsigned long long reseed_mode;   // PageRank reseed scatter: 0 push, 1 pull
+  Extrap ex;                        // extrapolation of the running series
 };
 
 // Persistent scratch of the update-batch path (grows, never shrinks), so a batch
@@ -208,6 +218,7 @@ struct suminc_ctx {
   uint64_t pr_state_id = 0;  // counts suminc_pr_init / suminc_pr_upload: a new PageRank state
   int pr_prec = SUMINC_PR_FP32_KAHAN;
   suminc::DevBuf pr_delta, pr_rank, pr_comp, pr_contrib;
+  suminc::DevBuf pr_prev;    // delta as the last round took it (the extrapolation's other point)
   suminc::DevBuf mass_part;  // block sums of the FP64 mass balance
   // pull mode: static chunk list of high in-degree vertices, rebuilt per graph version
   suminc::DevBuf pull_heavy, pull_short, pull_wave;

@@ -1,0 +1,134 @@
+"""Extrapolated delta series: wherever a run stops, rank and delta are a state of the
+same fixed point, r + (I - M)^-1 delta, and no graph takes more rounds than plain ones.
+
+Graphs: ones whose series lines up with one eigenvector (R-MAT, uniform, communities),
+ones that are eigenvectors from the start (ring, pairs) and ones that never line up
+(signed mass on a grid, a path, a ring), below and above a block of 1024 vertices.
+
+Tolerances against scipy's sparse solve: the stop rule's residual / (1 - d), plus rounding.
+FP64: 1e-12 of the state's mass.  FP32: a round rounds every delta to 2^-24, an
+extrapolation amplifies that by 1 + 2 beta <= 99 once, and (I - M)^-1 by 1 / (1 - d):
+2^-24 * (rounds + 99) / 0.15 of the mass at most, 1e-5 of it over 40 rounds and less
+where deltas shrink.
+"""
+import numpy as np
+import pytest
+import scipy.sparse as sp
+import scipy.sparse.linalg as sla
+
+from tests.conftest import DAMPING
+
+pytestmark = pytest.mark.gpu
+
+
+def graph(name):
+    rng = np.random.default_rng(7)
+    if name == "one":
+        n, u, v = 1, [], []
+    elif name == "ring":
+        n = 1025
+        u = np.arange(n)
+        v = (u + 1) % n
+    elif name == "pairs":
+        n = 1024
+        u = np.arange(n)
+        v = u ^ 1
+    elif name == "path":
+        n = 700
+        u = np.arange(n - 1)
+        v = u + 1
+    elif name == "grid":
+        a = 37
+        n = a * a
+        x, y = [t.ravel() for t in np.meshgrid(np.arange(a), np.arange(a))]
+        u = np.concatenate([(x * a + y)[(0 <= x + dx) & (x + dx < a) & (0 <= y + dy) & (y + dy < a)]
+                            for dx, dy in ((1, 0), (-1, 0), (0, 1), (0, -1))])
+        v = np.concatenate([((x + dx) * a + y + dy)[(0 <= x + dx) & (x + dx < a) & (0 <= y + dy) & (y + dy < a)]
+                            for dx, dy in ((1, 0), (-1, 0), (0, 1), (0, -1))])
+    elif name == "communities":
+        n, c = 5000, 100
+        u = rng.integers(0, n, 8 * n)
+        v = np.where(rng.random(8 * n) < 0.98, u // c * c + rng.integers(0, c, 8 * n), rng.integers(0, n, 8 * n))
+    elif name == "uniform":
+        n = 3001
+        u, v = rng.integers(0, n, 6 * n), rng.integers(0, n, 6 * n)
+    else:  # skewed ids, many vertices without out-edges
+        n = 4099
+        u, v = (n * rng.random(8 * n) ** 4).astype(int), (n * rng.random(8 * n) ** 3).astype(int)
+    key = np.unique(np.asarray(u, np.int64) * n + np.asarray(v, np.int64))
+    u, v = key // n, key % n
+    u, v = u[u != v], v[u != v]
+    off = np.zeros(n + 1, np.uint64)
+    off[1:] = np.cumsum(np.bincount(u, minlength=n))
+    return n, u, v, off
+
+
+def system(n, u, v):
+    deg = np.bincount(u, minlength=n) if len(u) else np.zeros(n)
+    return sp.csr_matrix((DAMPING / deg[u], (v, u)), shape=(n, n)) if len(u) else sp.csr_matrix((n, n))
+
+
+def plain_rounds(M, x, T):
+    """Rounds of the series with the activity rule: |delta| <= T / n waits."""
+    k = 0
+    while np.abs(x).sum() >= T:
+        a = np.where(np.abs(x) > T / len(x), x, 0.0)
+        x, k = x - a + M @ a, k + 1
+    return k
+
+
+def limit(M, r, x):
+    return r + sla.spsolve(sp.eye(M.shape[0], format="csc") - M.tocsc(), x)
+
+
+GRAPHS = ["one", "ring", "pairs", "path", "grid", "communities", "uniform", "skewed"]
+
+
+@pytest.mark.parametrize("seed", ["uniform", "vertex", "signed"])
+@pytest.mark.parametrize("name", GRAPHS)
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+def test_run_reaches_the_fixed_point(gpu, prec, name, seed):
+    n, u, v, off = graph(name)
+    M = system(n, u, v)
+    x = np.full(n, (1 - DAMPING) / n)
+    if seed == "vertex":
+        x = np.zeros(n)
+        x[0] = 1 - DAMPING
+    elif seed == "signed":
+        x = np.random.default_rng(3).standard_normal(n)
+        x *= 0.1 / np.abs(x).sum()
+    T = 1e-11 if prec == "fp64" else 1e-7
+    p = gpu.PR_FP64 if prec == "fp64" else gpu.PR_FP32_KAHAN
+    want = limit(M, np.zeros(n), x)
+    with gpu.Context(pr_precision=p, termcheck_threshold=T, max_rounds=1000) as ctx:
+        ctx.upload_csr(off, v.astype(np.uint32))
+        ctx.pr_upload(np.zeros(n), x)
+        st = ctx.pr_run()
+        r, d = ctx.pr_download()
+    mass = np.abs(x).sum()
+    assert st["residual"] < T
+    assert np.isclose(np.abs(d).sum(), st["residual"], rtol=1e-5, atol=T * 1e-5)
+    # one round more: FP32 sums may cross T a round later
+    assert st["rounds"] <= plain_rounds(M, x, T) + 1
+    assert np.abs(r - want).sum() <= T / (1 - DAMPING) + mass * (1e-12 if prec == "fp64" else 1e-5)
+
+
+@pytest.mark.parametrize("name", ["ring", "communities", "uniform", "skewed"])
+@pytest.mark.parametrize("cap", [1, 2, 3, 5, 8, 9, 10, 11, 12, 14])
+def test_round_cap_leaves_a_state_of_the_same_fixed_point(gpu, name, cap):
+    n, u, v, off = graph(name)
+    M = system(n, u, v)
+    x = np.full(n, (1 - DAMPING) / n)
+    want = limit(M, np.zeros(n), x)
+    with gpu.Context(pr_precision=gpu.PR_FP64, termcheck_threshold=1e-11, max_rounds=cap) as ctx:
+        ctx.upload_csr(off, v.astype(np.uint32))
+        ctx.pr_init()
+        st = ctx.pr_run(allow_not_converged=True)
+        r, d = ctx.pr_download()
+        # the (untaken) rest of an inactive vertex stays in delta, so the state is exact
+        assert np.abs(limit(M, r, d) - want).sum() < 1e-12
+        assert np.abs(d).sum() <= (1 - DAMPING) * DAMPING ** st["rounds"] * (1 + 1e-9)
+        ctx.set_params(max_rounds=1000)
+        ctx.pr_run()
+        r, _ = ctx.pr_download()
+    assert np.abs(r - want).sum() <= 1e-11 / (1 - DAMPING) + 1e-12
