@@ -121,6 +121,7 @@ struct Counters {
   unsigned long long bcopy[4];      // a batch's group counts, copied out with the counters
   unsigned long long reseed_mode;   // PageRank reseed scatter: 0 push, 1 pull
   Extrap ex;                        // extrapolation of the running series
+  unsigned long long pull_run;      // pull rounds in a row (sketch rounds)
 };
 
 // Persistent scratch of the update-batch path (grows, never shrinks), so a batch
@@ -181,6 +182,7 @@ struct Sketch {
   DevBuf sc_R, sc_D;         // PageRank rows (reach mass / residual) per entry
   DevBuf ss_dist;            // SSSP rows (in-cluster distance to every exit) per entry
   DevBuf bound, spnode;      // PageRank sketch accumulators
+  DevBuf ex_taken;           // inflow each exit turned into rank in the last round
   DevBuf xi_list, xi_count;  // internal edges leaving exits: (contribution slot of the exit, destination)
   DevBuf exits, exit_count;  // the exits of the current layout (sketch rounds' exit pass)
   DevBuf dead;               // K: cluster dissolved (its benefit fell to the threshold after batches)

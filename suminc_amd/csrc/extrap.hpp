@@ -23,6 +23,7 @@
 // path, signed mass on a regular grid) runs its plain rounds.
 #pragma once
 #include "ctx.hpp"
+#include "device.hpp"
 
 namespace suminc {
 
@@ -52,6 +53,66 @@ __device__ __forceinline__ double extrap_decide(Extrap& ex, double s1, double s2
 template <class T>
 __device__ __forceinline__ T extrap_value(T g, T p, double beta) {
   return (T)((double)g + beta * ((double)g - (double)p));
+}
+
+// rank[v] += x for an FP64 x: in FP32 mode the sum rank - comp is formed in FP64 and
+// split again, so a step several times the delta loses no more than a plain one.
+template <class T>
+__device__ __forceinline__ void rank_add_wide(T* rank, float* comp, uint32_t v, double x) {
+  if constexpr (sizeof(T) == 4) {
+    const double t = (double)rank[v] - (double)comp[v] + x;
+    const float r = (float)t;
+    rank[v] = r;
+    comp[v] = (float)((double)r - t);
+  } else {
+    rank[v] += x;
+  }
+}
+
+// Sums of a block's values of each of the K arrays of nparts (double or u64 bits per
+// kU bit k) into out[K], in a fixed order; all threads of a 1024-thread block.
+template <int K, unsigned kU>
+__device__ __forceinline__ void sum_parts(const double* __restrict__ partial, uint32_t nparts, double (*s)[K]) {
+  double acc[K];
+#pragma unroll
+  for (int k = 0; k < K; ++k) acc[k] = 0.0;  // the bits of u64 zero too
+  for (uint32_t i = threadIdx.x; i < nparts; i += 1024) {
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      const double x = partial[(size_t)k * nparts + i];
+      if (kU >> k & 1)
+        acc[k] = __longlong_as_double(__double_as_longlong(acc[k]) + __double_as_longlong(x));
+      else
+        acc[k] += x;
+    }
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      if (kU >> k & 1)
+        acc[k] = __longlong_as_double(__double_as_longlong(acc[k]) +
+                                      __shfl_xor((long long)__double_as_longlong(acc[k]), o));
+      else
+        acc[k] += __shfl_xor(acc[k], o);
+    }
+  }
+  if (lane_id() == 0) {
+#pragma unroll
+    for (int k = 0; k < K; ++k) s[threadIdx.x >> 6][k] = acc[k];
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int w = 1; w < 1024 / 64; ++w) {
+#pragma unroll
+      for (int k = 0; k < K; ++k) {
+        if (kU >> k & 1)
+          s[0][k] = __longlong_as_double(__double_as_longlong(s[0][k]) + __double_as_longlong(s[w][k]));
+        else
+          s[0][k] += s[w][k];
+      }
+    }
+  }
 }
 
 }  // namespace suminc

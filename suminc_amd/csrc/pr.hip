@@ -142,52 +142,6 @@ __device__ __forceinline__ void pr_round_end(Counters* cnt, unsigned long long a
   cnt->heavy_count = 0;
 }
 
-// Sums of a block's values of each of the K arrays of nparts (double or u64 bits per
-// kU bit k) into out[K], in a fixed order; all threads of a 1024-thread block.
-template <int K, unsigned kU>
-__device__ __forceinline__ void sum_parts(const double* __restrict__ partial, uint32_t nparts, double (*s)[K]) {
-  double acc[K];
-#pragma unroll
-  for (int k = 0; k < K; ++k) acc[k] = 0.0;  // the bits of u64 zero too
-  for (uint32_t i = threadIdx.x; i < nparts; i += 1024) {
-#pragma unroll
-    for (int k = 0; k < K; ++k) {
-      const double x = partial[(size_t)k * nparts + i];
-      if (kU >> k & 1)
-        acc[k] = __longlong_as_double(__double_as_longlong(acc[k]) + __double_as_longlong(x));
-      else
-        acc[k] += x;
-    }
-  }
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-#pragma unroll
-    for (int k = 0; k < K; ++k) {
-      if (kU >> k & 1)
-        acc[k] = __longlong_as_double(__double_as_longlong(acc[k]) +
-                                      __shfl_xor((long long)__double_as_longlong(acc[k]), o));
-      else
-        acc[k] += __shfl_xor(acc[k], o);
-    }
-  }
-  if (lane_id() == 0) {
-#pragma unroll
-    for (int k = 0; k < K; ++k) s[threadIdx.x >> 6][k] = acc[k];
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    for (int w = 1; w < 1024 / 64; ++w) {
-#pragma unroll
-      for (int k = 0; k < K; ++k) {
-        if (kU >> k & 1)
-          s[0][k] = __longlong_as_double(__double_as_longlong(s[0][k]) + __double_as_longlong(s[w][k]));
-        else
-          s[0][k] += s[w][k];
-      }
-    }
-  }
-}
-
 // Closes the round before (its active vertices are the fifth array of partials),
 // applies the stop rule and chooses the extrapolation and the scatter.
 __global__ void __launch_bounds__(1024) k_pr_decide(const double* __restrict__ partial, uint32_t nparts,
@@ -225,20 +179,6 @@ __device__ __forceinline__ void rank_add(T* rank, float* comp, uint32_t v, T x) 
     const float t = r + y;
     comp[v] = (t - r) - y;
     rank[v] = t;
-  } else {
-    rank[v] += x;
-  }
-}
-
-// rank[v] += x for an FP64 x: in FP32 mode the sum rank - comp is formed in FP64 and
-// split again, so a step several times the delta loses no more than a plain one.
-template <class T>
-__device__ __forceinline__ void rank_add_wide(T* rank, float* comp, uint32_t v, double x) {
-  if constexpr (sizeof(T) == 4) {
-    const double t = (double)rank[v] - (double)comp[v] + x;
-    const float r = (float)t;
-    rank[v] = r;
-    comp[v] = (float)((double)r - t);
   } else {
     rank[v] += x;
   }
@@ -663,6 +603,8 @@ __global__ void k_zero_counters(Counters* cnt) {
 // host side
 // ---------------------------------------------------------------------------
 unsigned push_grid() { return 2048; }
+
+void zero_counters(suminc_ctx* c) { k_zero_counters<<<1, 64, 0, c->stream>>>(dev_counters(c)); }
 
 // Contribution index of the plain pull: compact source positions when in use
 // (nullptr: vertex ids), and the CSC columns the plain pull reads.
@@ -2082,7 +2024,7 @@ void pr_run(suminc_ctx* c, suminc_stats* st) {
   const int max_rounds = c->prm.max_rounds > 0 ? c->prm.max_rounds : 1000000;
   const int div = c->prm.pull_threshold_div;
   if (div > 0) ensure_pull_heavy(c);
-  k_zero_counters<<<1, 64, 0, c->stream>>>(dev_counters(c));
+  zero_counters(c);
   SUMINC_HIP(hipEventRecord(c->ev_start, c->stream));
   // extrapolated runs take 8-16 rounds; one poll costs about as much as three empty rounds
   int group = 10;
@@ -2134,7 +2076,7 @@ void pr_step(suminc_ctx* c, double* residual) {
   const double T = c->prm.termcheck_threshold;
   const int div = c->prm.pull_threshold_div;
   if (div > 0) ensure_pull_heavy(c);
-  k_zero_counters<<<1, 64, 0, c->stream>>>(dev_counters(c));
+  zero_counters(c);
   // stop rule disabled for a single explicit step
   if (c->pr_prec == SUMINC_PR_FP64) enqueue_round<double>(c, T / c->n, -1.0, 1 << 30, div, 0, true);
   else enqueue_round<float>(c, T / c->n, -1.0, 1 << 30, div, 0, true);

@@ -21,6 +21,8 @@ void pr_upload(suminc_ctx* c, const double* rank, const double* delta);
 // FP64 mass balance of the current PageRank state into st->mass_total / mass_defect
 void pr_mass(suminc_ctx* c, suminc_stats* st);
 unsigned push_grid();
+// clears the device counters on the stream (the start of a run)
+void zero_counters(suminc_ctx* c);
 // positions of the vertices by decreasing degree (deg_off's row lengths; degree 0:
 // INF32) and cols (rows rows_off, up to m_cap entries) renamed to them; scratch
 // holds 16 B per vertex

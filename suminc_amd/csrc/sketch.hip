@@ -37,6 +37,7 @@
 
 #include "ctx.hpp"
 #include "device.hpp"
+#include "extrap.hpp"
 #include "pr.hpp"
 #include "push.hpp"
 #include "sketch.hpp"
@@ -1408,22 +1409,26 @@ struct SkArgs {
 };
 
 // residual of the sketch phase: |delta| of Single/entry vertices + |bound| of exits,
-// and the out-edges the round's senders will scatter (the push / pull choice).
-// kSkPer vertices a thread (vertex base + j * kBlock + t, coalesced).
+// and the out-edges the round's senders will scatter (the push / pull choice), block
+// sums in arrays of gridDim.x: the residual at 0, the edges (u64) at 1, and with a
+// candidate extrapolation (cnt->ex.cand > 0) the same of the extrapolated state at 2
+// and 3.  kSkPer vertices a thread (vertex base + j * kBlock + t, coalesced).
 constexpr int kSkPer = 4;
 template <class T>
 __global__ void __launch_bounds__(kBlock) k_sk_count(SkArgs a, const T* __restrict__ delta,
-                                                     const T* __restrict__ bound, double eps) {
-  __shared__ double s_sum[kBlock / 64];
-  __shared__ unsigned long long s_edges[kBlock / 64];
+                                                     const T* __restrict__ prev, const T* __restrict__ bound,
+                                                     double eps) {
+  __shared__ double s_sum[2][kBlock / 64];
+  __shared__ unsigned long long s_edges[2][kBlock / 64];
   if (a.cnt->done) return;
-  double x = 0;
-  unsigned long long ed = 0;
+  const double cand = a.cnt->ex.cand;
+  double x = 0, xx = 0;
+  unsigned long long ed = 0, edx = 0;
   const uint32_t base = blockIdx.x * (kBlock * kSkPer);
   // the kSkPer vertices' type, delta and row bounds loaded first (delta of a type
   // that holds none is read and ignored), then the sums
   uint8_t ty[kSkPer];
-  T dl[kSkPer];
+  T dl[kSkPer], pv[kSkPer];
   uint32_t o0[kSkPer], o1[kSkPer];
 #pragma unroll
   for (int j = 0; j < kSkPer; ++j) {
@@ -1434,17 +1439,29 @@ __global__ void __launch_bounds__(kBlock) k_sk_count(SkArgs a, const T* __restri
     o0[j] = in ? a.off[v] : 0u;
     o1[j] = in ? a.off[v + 1] : 0u;
   }
+  if (cand > 0.0) {
+#pragma unroll
+    for (int j = 0; j < kSkPer; ++j) {
+      const uint32_t v = base + j * kBlock + threadIdx.x;
+      pv[j] = v < a.n ? prev[v] : T(0);
+    }
+  }
 #pragma unroll
   for (int j = 0; j < kSkPer; ++j) {
     const uint32_t v = base + j * kBlock + threadIdx.x;
     const uint8_t t = ty[j];
     if (t == 4) continue;
     const uint32_t deg = o1[j] - o0[j];
-    double dv = 0;
+    double dv = 0, dx = 0;
     if (t != 1) {
       dv = (double)fabs_t(dl[j]);
       x += dv;
       if (t == 0 && dv > eps) ed += deg;
+      if (cand > 0.0) {
+        dx = (double)fabs_t(extrap_value<T>(dl[j], pv[j], cand));
+        xx += dx;
+        if (t == 0 && dx > eps) edx += deg;
+      }
     }
     if (t == 1 || t == 3) {
       const double b = (double)fabs_t(bound[v]);
@@ -1452,64 +1469,75 @@ __global__ void __launch_bounds__(kBlock) k_sk_count(SkArgs a, const T* __restri
       // an exit sends in the round its cluster's entries inject: its own entry's
       // mass (a BothOutIn hub's) leaves it this round
       if (b > eps || (t == 3 && dv > eps)) ed += deg;
+      if (cand > 0.0) {
+        xx += b;  // the rounds a step follows leave no inflow behind (k_sk_decide)
+        if (b > eps || (t == 3 && dx > eps)) edx += deg;
+      }
     }
   }
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) {
     x += __shfl_xor(x, o);
     ed += __shfl_xor(ed, o);
+    xx += __shfl_xor(xx, o);
+    edx += __shfl_xor(edx, o);
   }
   if (lane_id() == 0) {
-    s_sum[threadIdx.x >> 6] = x;
-    s_edges[threadIdx.x >> 6] = ed;
+    s_sum[0][threadIdx.x >> 6] = x;
+    s_edges[0][threadIdx.x >> 6] = ed;
+    s_sum[1][threadIdx.x >> 6] = xx;
+    s_edges[1][threadIdx.x >> 6] = edx;
   }
   __syncthreads();
-  if (threadIdx.x == 0) {
+  if (threadIdx.x < 2) {
     double t = 0;
     unsigned long long te = 0;
     for (int w = 0; w < kBlock / 64; ++w) {
-      t += s_sum[w];
-      te += s_edges[w];
+      t += s_sum[threadIdx.x][w];
+      te += s_edges[threadIdx.x][w];
     }
-    a.partial[blockIdx.x] = t;
-    reinterpret_cast<unsigned long long*>(a.partial)[2 * gridDim.x + blockIdx.x] = te;
+    const size_t at = (size_t)threadIdx.x * 2 * gridDim.x + blockIdx.x;
+    a.partial[at] = t;
+    reinterpret_cast<unsigned long long*>(a.partial)[at + gridDim.x] = te;
   }
 }
 
-// Stop rule of the sketch phase and the round's scatter: pull over the CSC when
-// the senders' out-edges exceed m / div (as the plain rounds decide), else push.
-__global__ void __launch_bounds__(1024) k_sk_decide(const double* __restrict__ partial, uint32_t nparts, Counters* cnt,
-                                                    double T, int max_rounds, uint64_t m, int div,
-                                                    uint8_t* __restrict__ mode_hist) {
-  __shared__ double s[1024];
-  __shared__ unsigned long long se[1024];
+// Closes the round before (the edges that its senders and exits scattered), then the
+// stop rule of the sketch phase, the extrapolation (extrap.hpp) and the round's scatter:
+// pull over the CSC when the senders' out-edges exceed m / div (as the plain rounds
+// decide), else push.  An extrapolation scales what the last round took, the exits'
+// inflow included, and leaves their inflow as it is, so it needs none of it to have
+// been left behind by that round or the one before: both were pulls (their exit pass
+// takes every inflow).  A 1% batch on R-MAT of 2^24 vertices (201M edges), batch, query
+// and read-back: 58 sketch rounds, 94.3 ms -> 53.0 ms with the steps; off the FP64 ranks
+// by 9.4e-8 instead of 1.6e-6.
+__global__ void __launch_bounds__(1024) k_sk_decide(const double* __restrict__ partial, uint32_t nparts,
+                                                    uint32_t nexit_parts, Counters* cnt, double T, int max_rounds,
+                                                    uint64_t m, int div, uint8_t* __restrict__ mode_hist) {
+  __shared__ double s[1024 / 64][5], se[1024 / 64][1];
   if (cnt->done) return;
-  const unsigned long long* pe = reinterpret_cast<const unsigned long long*>(partial) + 2 * nparts;
-  double acc = 0;
-  unsigned long long acc_e = 0;
-  for (uint32_t i = threadIdx.x; i < nparts; i += 1024) {
-    acc += partial[i];
-    acc_e += pe[i];
-  }
-  s[threadIdx.x] = acc;
-  se[threadIdx.x] = acc_e;
-  __syncthreads();
-  for (int o = 512; o > 0; o >>= 1) {
-    if (threadIdx.x < o) {
-      s[threadIdx.x] += s[threadIdx.x + o];
-      se[threadIdx.x] += se[threadIdx.x + o];
-    }
-    __syncthreads();
-  }
+  sum_parts<5, 0b11010u>(partial, nparts, s);
+  sum_parts<1, 0b1u>(partial + (size_t)5 * nparts, nexit_parts, se);
   if (threadIdx.x == 0) {
-    double r = s[0];
+    if (cnt->rounds) {
+      cnt->edges += (unsigned long long)(__double_as_longlong(s[0][4]) + __double_as_longlong(se[0][0]));
+      cnt->wl_count[0] = 0;
+      cnt->wl_count[1] = 0;
+      cnt->heavy_count = 0;
+      cnt->pull_run = cnt->mode ? cnt->pull_run + 1 : 0;
+    }
+    if (cnt->pull_run < 2) cnt->ex.cand = 0.0;
+    const double s1 = s[0][0];
+    const double r = extrap_decide(cnt->ex, s1, s[0][2], T);
+    const unsigned long long edges = (unsigned long long)__double_as_longlong(cnt->ex.beta > 0.0 ? s[0][3] : s[0][1]);
+    cnt->round_edges = 0;
     cnt->residual = r;
-    if (r != r || r > 1e300) cnt->aux[0] = 1;
+    if (s1 != s1 || s1 > 1e300) cnt->aux[0] = 1;
     if (!(r >= T) || (long long)cnt->rounds >= (long long)max_rounds || cnt->aux[0]) {
       cnt->done = 1;
       return;
     }
-    cnt->mode = div > 0 && se[0] * (unsigned long long)div > m ? 1 : 0;
+    cnt->mode = div > 0 && edges * (unsigned long long)div > m ? 1 : 0;
     if (cnt->rounds < 65536) mode_hist[cnt->rounds] = (uint8_t)cnt->mode;
     cnt->rounds += 1;
   }
@@ -1522,8 +1550,10 @@ __global__ void __launch_bounds__(1024) k_sk_decide(const double* __restrict__ p
 // of the cluster, so mass crosses a cluster within the round it entered (an order
 // the reference's parallel loop may take as well).  The flush at the end of the
 // sketch phase is the exit pass over every non-zero inflow.
-// Block sums of the round's edges: k_sk_send in partial[g, 2g) (u64 view, g its
-// grid), k_sk_exits in partial[2g, 2g + its grid) (the count's slots, read by then).
+// Block sums of the round's edges (u64 view): k_sk_send in partial[4g, 5g), g its grid
+// and the count's, k_sk_exits in partial[5g, 5g + its grid).  A chosen extrapolation
+// (cnt->ex.beta) is applied first: by k_sk_send to delta and to what Singles (rank)
+// and entries (spnode) took, by k_sk_exits to what the exits took (ex_taken).
 template <class T>
 __device__ __forceinline__ void sk_contrib(const SkArgs& a, T* contrib, uint32_t v, T x) {
   const uint32_t slot = a.pos ? a.pos[v] : v;  // vertices without out-edges have no position and never send
@@ -1545,12 +1575,14 @@ __device__ __forceinline__ void sk_block_edges(unsigned long long ed, unsigned l
 }
 
 template <class T>
-__global__ void __launch_bounds__(kBlock) k_sk_send(SkArgs a, T* __restrict__ delta, T* __restrict__ spnode,
+__global__ void __launch_bounds__(kBlock) k_sk_send(SkArgs a, T* __restrict__ delta, T* __restrict__ prev,
+                                                    T* __restrict__ spnode,
                                                     T* __restrict__ rank, float* __restrict__ comp,
                                                     T* __restrict__ wl_c, T* __restrict__ sc_x,
                                                     T* __restrict__ contrib, double eps, T d) {
   if (a.cnt->done) return;
   const bool pull = a.cnt->mode != 0;  // contributions for the CSC pull instead of push items
+  const double beta = a.cnt->ex.beta;
   const uint32_t base = blockIdx.x * (kBlock * kSkPer);
   unsigned long long ed = 0;
   // the kSkPer vertices' type, delta and row bounds loaded first
@@ -1577,6 +1609,19 @@ __global__ void __launch_bounds__(kBlock) k_sk_send(SkArgs a, T* __restrict__ de
     if (v < a.n) {
       const uint8_t t = ty[j];
       deg = o1[j] - o0[j];
+      if (t == 0 || t == 2 || t == 3) {
+        if (beta > 0.0) {
+          const T p = prev[v];
+          const T x = extrap_value<T>(dl[j], p, beta);
+          if ((double)fabs_t(p) > eps) {
+            if (t == 0) rank_add_wide<T>(rank, comp, v, beta * (double)p);
+            else spnode[v] = (T)((double)spnode[v] + beta * (double)p);
+          }
+          if (!((double)fabs_t(x) > eps)) delta[v] = x;
+          dl[j] = x;
+        }
+        prev[v] = dl[j];
+      }
       if (t == 0) {  // SingleNode: plain push over its out-list
         const T dv = dl[j];
         if ((double)fabs_t(dv) > eps) {
@@ -1600,19 +1645,21 @@ __global__ void __launch_bounds__(kBlock) k_sk_send(SkArgs a, T* __restrict__ de
     push_item<T>(want_push && !pull, v, cval, deg, a.wl_v, wl_c, a.heavy, a.cnt);
     if (want_push) ed += deg;
   }
-  sk_block_edges<T>(ed, reinterpret_cast<unsigned long long*>(a.partial) + gridDim.x + blockIdx.x);
+  sk_block_edges<T>(ed, reinterpret_cast<unsigned long long*>(a.partial) + (size_t)4 * gridDim.x + blockIdx.x);
 }
 
-// The exits of the current layout, one per thread (flush: every non-zero inflow).
+// The exits of the current layout, one per thread (flush: every non-zero inflow, and
+// the pending extrapolation of the exits is k_sk_extrap_end's).
 template <class T>
 __global__ void __launch_bounds__(kBlock) k_sk_exits(SkArgs a, const uint32_t* __restrict__ exits,
                                                      const unsigned long long* __restrict__ n_exits,
                                                      T* __restrict__ bound, T* __restrict__ rank,
-                                                     float* __restrict__ comp, T* __restrict__ wl_c,
-                                                     T* __restrict__ contrib, double eps, T d, int flush,
-                                                     uint32_t part_base) {
+                                                     float* __restrict__ comp, T* __restrict__ taken,
+                                                     T* __restrict__ wl_c, T* __restrict__ contrib, double eps, T d,
+                                                     int flush, uint32_t part_base) {
   if (a.cnt->done) return;
   const bool pull = a.cnt->mode != 0;
+  const double beta = flush ? 0.0 : a.cnt->ex.beta;
   const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
   bool want_push = false;
   T cval = T(0);
@@ -1621,7 +1668,11 @@ __global__ void __launch_bounds__(kBlock) k_sk_exits(SkArgs a, const uint32_t* _
     v = exits[i];
     deg = a.off[v + 1] - a.off[v];
     const T b = bound[v];
-    if (flush ? b != T(0) : (double)fabs_t(b) > eps) {
+    if (beta > 0.0 && taken[i] != T(0)) rank_add_wide<T>(rank, comp, v, beta * (double)taken[i]);
+    // a pull sends every exit's inflow at no cost, so it leaves none behind
+    const bool take = flush || pull ? b != T(0) : (double)fabs_t(b) > eps;
+    if (!flush) taken[i] = take ? b : T(0);
+    if (take) {
       bound[v] = T(0);
       kahan_add(rank, comp, v, b);
       // the push skips an exit's edges inside its cluster; the pull takes them back
@@ -1685,24 +1736,30 @@ __global__ void __launch_bounds__(kBlock) k_sk_shortcut(uint32_t E, const T* __r
   }
 }
 
-__global__ void __launch_bounds__(1024) k_sk_end(Counters* cnt, const unsigned long long* __restrict__ pe,
-                                                 uint32_t nparts) {
-  __shared__ unsigned long long s[1024];
-  if (cnt->done) return;
-  unsigned long long acc = 0;
-  for (uint32_t i = threadIdx.x; i < nparts; i += 1024) acc += pe[i];
-  s[threadIdx.x] = acc;
-  __syncthreads();
-  for (int o = 512; o > 0; o >>= 1) {
-    if (threadIdx.x < o) s[threadIdx.x] += s[threadIdx.x + o];
-    __syncthreads();
+// Applies an extrapolation that was chosen by the decision that ended the sketch phase.
+template <class T>
+__global__ void __launch_bounds__(kBlock) k_sk_extrap_end(SkArgs a, T* __restrict__ delta, const T* __restrict__ prev,
+                                                          T* __restrict__ spnode, T* __restrict__ rank,
+                                                          float* __restrict__ comp, double eps, double beta) {
+  const uint32_t v = blockIdx.x * kBlock + threadIdx.x;
+  if (v >= a.n) return;
+  const uint8_t t = a.ntype[v];
+  if (t == 1 || t == 4) return;
+  const T p = prev[v];
+  delta[v] = extrap_value<T>(delta[v], p, beta);
+  if ((double)fabs_t(p) > eps) {
+    if (t == 0) rank_add_wide<T>(rank, comp, v, beta * (double)p);
+    else spnode[v] = (T)((double)spnode[v] + beta * (double)p);
   }
-  if (threadIdx.x) return;
-  cnt->edges += s[0];
-  cnt->round_edges = 0;
-  cnt->wl_count[0] = 0;
-  cnt->wl_count[1] = 0;
-  cnt->heavy_count = 0;
+}
+
+template <class T>
+__global__ void __launch_bounds__(kBlock) k_sk_extrap_exits(const uint32_t* __restrict__ exits,
+                                                            const unsigned long long* __restrict__ n_exits,
+                                                            const T* __restrict__ taken, T* __restrict__ rank,
+                                                            float* __restrict__ comp, double beta) {
+  const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
+  if (i < *n_exits && taken[i] != T(0)) rank_add_wide<T>(rank, comp, exits[i], beta * (double)taken[i]);
 }
 
 // push list of a flush/precompute pass: run once, then clear
@@ -1912,6 +1969,7 @@ static void sum_pr_run_t(suminc_ctx* c, suminc_stats* st) {
   suminc_stats out{};
   SUMINC_HIP(hipEventRecord(c->ev_start, c->stream));
   // 1. precompute of dirty clusters + the exits' sends
+  zero_counters(c);
   k_lists_clear<<<1, 64, 0, c->stream>>>(cnt);
   if (s.K)
     k_sk_precompute<T><<<s.K, kBlock, 0, c->stream>>>(a, s.cl_off.as<uint32_t>(), s.cl_mem.as<uint32_t>(),
@@ -1936,14 +1994,16 @@ static void sum_pr_run_t(suminc_ctx* c, suminc_stats* st) {
   const unsigned g4 = grid_for(n, kBlock * kSkPer);  // the vertex passes: kSkPer vertices a thread
   const unsigned ge = grid_for(n_exits);             // the exit pass
   c->tmp4.ensure(65536);  // per-round scatter mode (profile attribution)
-  int group = 4;
+  s.ex_taken.ensure(n_exits * es + es);
+  int group = 10;  // as the plain rounds
   size_t slot = 0;
   while (true) {
     for (int i = 0; i < group; ++i, ++slot) {
-      k_sk_count<T><<<g4, kBlock, 0, c->stream>>>(a, c->pr_delta.as<T>(), s.bound.as<T>(), eps);
-      k_sk_decide<<<1, 1024, 0, c->stream>>>(a.partial, g4, cnt, T_stop, max_rounds, c->m, div,
+      k_sk_count<T><<<g4, kBlock, 0, c->stream>>>(a, c->pr_delta.as<T>(), c->pr_prev.as<T>(), s.bound.as<T>(), eps);
+      k_sk_decide<<<1, 1024, 0, c->stream>>>(a.partial, g4, ge, cnt, T_stop, max_rounds, c->m, div,
                                              c->tmp4.as<uint8_t>());
-      k_sk_send<T><<<g4, kBlock, 0, c->stream>>>(a, c->pr_delta.as<T>(), s.spnode.as<T>(), c->pr_rank.as<T>(),
+      k_sk_send<T><<<g4, kBlock, 0, c->stream>>>(a, c->pr_delta.as<T>(), c->pr_prev.as<T>(), s.spnode.as<T>(),
+                                                 c->pr_rank.as<T>(),
                                                  c->pr_comp.as<float>(), c->wl1.as<T>(), c->tmp3.as<T>(),
                                                  c->pr_contrib.as<T>(), eps, d);
       k_sk_shortcut<T><<<grid_for(s.E, kBlock, push_grid()), kBlock, 0, c->stream>>>(
@@ -1952,7 +2012,8 @@ static void sum_pr_run_t(suminc_ctx* c, suminc_stats* st) {
           s.sc_base.as<unsigned long long>(), s.sc_R.as<T>(), s.bound.as<T>());
       k_sk_exits<T><<<ge, kBlock, 0, c->stream>>>(a, s.exits.as<uint32_t>(), s.exit_count.as<unsigned long long>(),
                                                   s.bound.as<T>(), c->pr_rank.as<T>(), c->pr_comp.as<float>(),
-                                                  c->wl1.as<T>(), c->pr_contrib.as<T>(), eps, d, 0, 2 * g4);
+                                                  s.ex_taken.as<T>(), c->wl1.as<T>(), c->pr_contrib.as<T>(), eps, d,
+                                                  0, 5 * g4);
       sk_push_pass<T>(c);
       if (c->prof_on) SUMINC_HIP(hipEventRecord(prof_event(c, 2 * slot), c->stream));
       if (div > 0) pull_scatter<T>(c, 0);
@@ -1961,12 +2022,11 @@ static void sum_pr_run_t(suminc_ctx* c, suminc_stats* st) {
         k_pull_unskip<T><<<grid_for(s.ie_m + 1, kBlock, 4096), kBlock, 0, c->stream>>>(
             s.xi_list.as<uint2>(), s.xi_count.as<unsigned long long>(), c->pr_contrib.as<T>(), c->pr_delta.as<T>(),
             cnt);
-      k_sk_end<<<1, 1024, 0, c->stream>>>(cnt, reinterpret_cast<unsigned long long*>(a.partial) + g4, g4 + ge);
     }
     SUMINC_HIP(hipGetLastError());
     read_counters(c);
     if (c->host_counters->done) break;
-    if (group < 32) group *= 2;
+    group = slot < 20 ? 4 : std::min(32, 2 * group);
   }
   const Counters* h = c->host_counters;
   out.sketch_rounds = (double)h->rounds;  // sketch rounds
@@ -1989,11 +2049,19 @@ static void sum_pr_run_t(suminc_ctx* c, suminc_stats* st) {
     }
   }
   SUMINC_REQUIRE(!h->aux[0], SUMINC_E_NUMERIC, "NaN/Inf in the sketch residual");
+  if (h->ex.beta > 0.0) {
+    k_sk_extrap_end<T><<<grid_for(n), kBlock, 0, c->stream>>>(a, c->pr_delta.as<T>(), c->pr_prev.as<T>(),
+                                                             s.spnode.as<T>(), c->pr_rank.as<T>(),
+                                                             c->pr_comp.as<float>(), eps, h->ex.beta);
+    k_sk_extrap_exits<T><<<ge, kBlock, 0, c->stream>>>(s.exits.as<uint32_t>(),
+                                                       s.exit_count.as<unsigned long long>(), s.ex_taken.as<T>(),
+                                                       c->pr_rank.as<T>(), c->pr_comp.as<float>(), h->ex.beta);
+  }
   // 3. flush the exits' pending inflow, 4. correction
   k_lists_clear<<<1, 64, 0, c->stream>>>(cnt);
   k_sk_exits<T><<<ge, kBlock, 0, c->stream>>>(a, s.exits.as<uint32_t>(), s.exit_count.as<unsigned long long>(),
                                               s.bound.as<T>(), c->pr_rank.as<T>(), c->pr_comp.as<float>(),
-                                              c->wl1.as<T>(), c->pr_contrib.as<T>(), eps, d, 1, 2 * g4);
+                                              s.ex_taken.as<T>(), c->wl1.as<T>(), c->pr_contrib.as<T>(), eps, d, 1, 5 * g4);
   sk_push_pass<T>(c);
   k_lists_clear<<<1, 64, 0, c->stream>>>(cnt);
   if (s.K)

@@ -132,3 +132,56 @@ def test_round_cap_leaves_a_state_of_the_same_fixed_point(gpu, name, cap):
         ctx.pr_run()
         r, _ = ctx.pr_download()
     assert np.abs(r - want).sum() <= 1e-11 / (1 - DAMPING) + 1e-12
+
+
+def hubs(n=6007, hubs=300):
+    """A skewed core over `hubs` vertices; the others hang on one of them, most both ways."""
+    rng = np.random.default_rng(11)
+    u, v = (hubs * rng.random(8 * hubs) ** 2).astype(int), (hubs * rng.random(8 * hubs) ** 2).astype(int)
+    leaf = np.arange(hubs, n)
+    h = rng.integers(0, hubs, len(leaf))
+    back = rng.random(len(leaf)) < 0.8
+    key = np.unique(np.concatenate([u * n + v, leaf * n + h, (h * n + leaf)[back]]).astype(np.int64))
+    u, v = key // n, key % n
+    u, v = u[u != v], v[u != v]
+    off = np.zeros(n + 1, np.uint64)
+    off[1:] = np.cumsum(np.bincount(u, minlength=n))
+    return n, u, v, off
+
+
+@pytest.mark.parametrize("div", [3, 1_000_000, 0], ids=["mixed", "pull", "push"])
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+def test_sketch_run_reaches_the_fixed_point(gpu, prec, div):
+    """From scratch, from a signed state and at round caps, over supernodes: the exits'
+    and entries' share of an extrapolation step (pull rounds), and none of it (push)."""
+    n, u, v, off = hubs()
+    M = system(n, u, v)
+    T = 1e-11 if prec == "fp64" else 1e-7
+    tol = 1e-12 if prec == "fp64" else 1e-5
+    p = gpu.PR_FP64 if prec == "fp64" else gpu.PR_FP32_KAHAN
+    x0 = np.full(n, (1 - DAMPING) / n)
+    x1 = np.random.default_rng(5).standard_normal(n)
+    x1 *= 0.1 / np.abs(x1).sum()
+    with gpu.Context(pr_precision=p, termcheck_threshold=T, max_rounds=1000, pull_threshold_div=div) as ctx:
+        ctx.upload_csr(off, v.astype(np.uint32))
+        ctx.cluster_leaves(1024, 2)
+        for x in (x0, x1):
+            info = ctx.sum_build(2, 1024, 1.0)  # a fresh build: every cluster runs its precompute
+            assert info["clusters"] > 100 and info["entries"] > 100
+            want = limit(M, np.zeros(n), x)
+            ctx.pr_upload(np.zeros(n), x)
+            st = ctx.sum_pr_run()
+            r, _ = ctx.pr_download()
+            assert st["residual"] < T
+            assert st["sketch_rounds"] + st["residual_rounds"] <= plain_rounds(M, x, T) + 3
+            assert np.abs(r - want).sum() <= T / (1 - DAMPING) + 0.15 * tol
+        want = limit(M, np.zeros(n), x0)
+        for cap in (4, 7, 9, 12):
+            ctx.set_params(max_rounds=cap)
+            ctx.pr_upload(np.zeros(n), x0)
+            try:
+                ctx.sum_pr_run()
+            except gpu.SumincError as e:
+                assert e.code == gpu.E_NOT_CONVERGED
+            r, d = ctx.pr_download()
+            assert np.abs(limit(M, r, d) - want).sum() <= 0.15 * tol
