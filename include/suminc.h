@@ -476,7 +476,7 @@ int suminc_compress_mirror_load(suminc_ctx* ctx, const char* path, suminc_compre
  * termcheck_threshold.  Backward for L = sum_i c_i r_i: the same series on the
  * transpose graph from mu_0 = c, stopped when sum|mu| < termcheck_threshold * sum|c|,
  * gives lambda; dL/dp = (1-d) lambda, dL/dw_uv = (d r_u / s_u)(lambda_v - sum_k W[u,k]
- * lambda_k).  State in FP32 with Kahan sums or FP64 (pr_precision).  Vectors are n
+ * lambda_k).  A series may take extrapolation steps, as suminc_pr_run does.  State in FP32 with Kahan sums or FP64 (pr_precision).  Vectors are n
  * floats, edge weights and their gradient m floats in out-CSR order; every pointer
  * may be host or device memory of the context's GPU.  All four synchronise.
  * suminc_wpr_backward differentiates the context's last forward (its rank and

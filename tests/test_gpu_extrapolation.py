@@ -185,3 +185,41 @@ def test_sketch_run_reaches_the_fixed_point(gpu, prec, div):
                 assert e.code == gpu.E_NOT_CONVERGED
             r, d = ctx.pr_download()
             assert np.abs(limit(M, r, d) - want).sum() <= 0.15 * tol
+
+
+@pytest.mark.parametrize("name", ["ring", "path", "grid", "communities", "uniform", "skewed"])
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+def test_weighted_series_and_adjoint(gpu, prec, name):
+    """Forward from one vertex and adjoint from signed loss weights (the transpose does
+    not contract the 1-norm) against solves of both systems."""
+    n, u, v, off = graph(name)
+    rng = np.random.default_rng(9)
+    w = (1.0 - rng.random(len(u))).astype(np.float32)
+    s = np.bincount(u, weights=w.astype(float), minlength=n)
+    M = sp.csr_matrix((DAMPING * w / s[u], (v, u)), shape=(n, n))
+    p = np.zeros(n, np.float32)
+    p[0] = 1.0
+    c = rng.standard_normal(n).astype(np.float32)
+    T = 1e-11 if prec == "fp64" else 1e-7
+    tol = 1e-6 if prec == "fp64" else 1e-5  # rank and gradients come back as FP32
+    pr = gpu.PR_FP64 if prec == "fp64" else gpu.PR_FP32_KAHAN
+    with gpu.Context(pr_precision=pr, termcheck_threshold=T, max_rounds=2000) as ctx:
+        ctx.upload_csr(off, v.astype(np.uint32), w)
+        ctx.wpr_set_weights(w)
+        r, st = ctx.wpr_forward(p)
+        gp, gw, sb = ctx.wpr_backward(c)
+    want = limit(M, np.zeros(n), (1 - DAMPING) * p.astype(float))
+    lam = limit(M.T.tocsr(), np.zeros(n), c.astype(float))
+    assert st["rounds"] <= max(1, plain_rounds_all(M, (1 - DAMPING) * p.astype(float), T)) + 1
+    assert sb["rounds"] <= max(1, plain_rounds_all(M.T.tocsr(), c.astype(float), T * np.abs(c).sum())) + 1
+    assert np.abs(r - want).sum() <= T / (1 - DAMPING) + tol
+    gw_want = (want / np.where(s > 0, s, 1))[u] * (DAMPING * lam[v] - (M.T @ lam)[u])
+    assert np.abs(gp - (1 - DAMPING) * lam).max() <= tol * np.abs(lam).max()
+    assert np.abs(gw - gw_want).max() <= tol * max(np.abs(gw_want).max(), np.abs(lam).max() * (want[u] / s[u]).max())
+
+
+def plain_rounds_all(M, x, T):
+    k = 0
+    while np.abs(x).sum() >= T:
+        x, k = M @ x, k + 1
+    return k
