@@ -5,6 +5,7 @@
 
 #include "ctx.hpp"
 #include "pr.hpp"
+#include "readback.hpp"
 #include "sketch.hpp"
 
 namespace suminc {
@@ -107,6 +108,7 @@ int suminc_ctx_create(int device, const suminc_params* params, suminc_ctx** out)
   suminc_ctx* c = new (std::nothrow) suminc_ctx();
   if (!c) return SUMINC_E_NOMEM;
   c->device = device;
+  readback_context(1);
   int rc = guarded(c, [&] {
     int count = 0;
     SUMINC_HIP(hipGetDeviceCount(&count));
@@ -153,6 +155,7 @@ int suminc_ctx_destroy(suminc_ctx* c) {
   wpr_release(c);
   rsk_release(c);
   mirror_release(c);
+  readback_context(-1);
   delete c;  // DevBuf destructors free device memory
   if (s) (void)hipStreamDestroy(s);
   return SUMINC_OK;

@@ -43,6 +43,7 @@
 #include "device.hpp"
 #include "extrap.hpp"
 #include "pr.hpp"
+#include "readback.hpp"
 #include "push.hpp"
 
 namespace suminc {
@@ -511,15 +512,15 @@ __global__ void k_pr_init(uint32_t n, T* delta, T* rank, float* comp, T init_del
   if (comp) comp[v] = 0.f;
 }
 
+// FP64 copies of n values: the ranks (rank - comp) or, comp null, x as it is
 template <class T>
-__global__ void k_pr_to_f64(uint32_t n, const T* delta, const T* rank, const float* comp, double* d_out,
-                            double* r_out) {
-  uint32_t v = blockIdx.x * blockDim.x + threadIdx.x;
+__global__ void __launch_bounds__(kBlock) k_pr_to_f64(uint32_t n, const T* __restrict__ x, const float* __restrict__ comp,
+                                                      double* __restrict__ out) {
+  const uint32_t v = blockIdx.x * kBlock + threadIdx.x;
   if (v >= n) return;
-  d_out[v] = (double)delta[v];
-  double r = (double)rank[v];
+  double r = (double)x[v];
   if (comp) r -= (double)comp[v];
-  r_out[v] = r;
+  out[v] = r;
 }
 
 template <class T>
@@ -2088,20 +2089,26 @@ void pr_step(suminc_ctx* c, double* residual) {
 
 void pr_download(suminc_ctx* c, double* rank, double* delta) {
   SUMINC_REQUIRE(c->pr_ready, SUMINC_E_STATE, "PageRank state not initialised");
-  DevBuf dd, dr;
-  dd.ensure((size_t)c->n * 8);
-  dr.ensure((size_t)c->n * 8);
-  if (c->pr_prec == SUMINC_PR_FP64)
-    k_pr_to_f64<double><<<grid_for(c->n), kBlock, 0, c->stream>>>(c->n, c->pr_delta.as<double>(),
-                                                                 c->pr_rank.as<double>(), nullptr,
-                                                                 dd.as<double>(), dr.as<double>());
-  else
-    k_pr_to_f64<float><<<grid_for(c->n), kBlock, 0, c->stream>>>(c->n, c->pr_delta.as<float>(),
-                                                                c->pr_rank.as<float>(), c->pr_comp.as<float>(),
-                                                                dd.as<double>(), dr.as<double>());
-  SUMINC_HIP(hipGetLastError());
-  if (rank) SUMINC_HIP(hipMemcpyAsync(rank, dr.p, (size_t)c->n * 8, hipMemcpyDeviceToHost, c->stream));
-  if (delta) SUMINC_HIP(hipMemcpyAsync(delta, dd.p, (size_t)c->n * 8, hipMemcpyDeviceToHost, c->stream));
+  auto convert = [c](int part, uint64_t first, uint64_t count, void* out) {
+    const unsigned g = grid_for(count);
+    const DevBuf& x = part == 0 ? c->pr_rank : c->pr_delta;
+    double* to = reinterpret_cast<double*>(out);
+    if (c->pr_prec == SUMINC_PR_FP64)
+      k_pr_to_f64<double><<<g, kBlock, 0, c->stream>>>((uint32_t)count, x.as<double>() + first, nullptr, to);
+    else
+      k_pr_to_f64<float><<<g, kBlock, 0, c->stream>>>((uint32_t)count, x.as<float>() + first,
+                                                     part == 0 ? c->pr_comp.as<float>() + first : nullptr, to);
+  };
+  if (readback(c, {{rank, c->n, 8}, {delta, c->n, 8}}, convert)) return;
+  DevBuf tmp;
+  tmp.ensure((size_t)c->n * 8);
+  double* dst[2] = {rank, delta};
+  for (int k = 0; k < 2; ++k) {
+    if (!dst[k]) continue;
+    convert(k, 0, c->n, tmp.p);
+    SUMINC_HIP(hipGetLastError());
+    SUMINC_HIP(hipMemcpyAsync(dst[k], tmp.p, (size_t)c->n * 8, hipMemcpyDeviceToHost, c->stream));
+  }
   SUMINC_HIP(hipStreamSynchronize(c->stream));
 }
 

@@ -21,6 +21,7 @@
 #include "ctx.hpp"
 #include "device.hpp"
 #include "pr.hpp"
+#include "readback.hpp"
 
 namespace suminc {
 
@@ -160,12 +161,14 @@ __global__ void k_sssp_begin(Counters* cnt, unsigned long long* seeds) {
   cnt->edges = 0;
 }
 
-__global__ void k_sssp_unpack(uint32_t n, const unsigned long long* dp, int app, uint32_t* dist, uint32_t* parent) {
-  uint32_t v = blockIdx.x * blockDim.x + threadIdx.x;
+// one half of the words of n vertices: the parents, or the values of the app
+__global__ void __launch_bounds__(kBlock) k_sssp_unpack(uint32_t n, const unsigned long long* __restrict__ dp, int app,
+                                                        int parent, uint32_t* __restrict__ out) {
+  const uint32_t v = blockIdx.x * kBlock + threadIdx.x;
   if (v >= n) return;
-  unsigned long long x = dp[v];
-  dist[v] = app == SUMINC_APP_SSWP ? ~(uint32_t)(x >> 32) : (uint32_t)(x >> 32);
-  parent[v] = (uint32_t)x;
+  const unsigned long long x = dp[v];
+  const uint32_t hi = (uint32_t)(x >> 32);
+  out[v] = parent ? (uint32_t)x : app == SUMINC_APP_SSWP ? ~hi : hi;
 }
 
 SsspArgs sssp_args(suminc_ctx* c) {
@@ -314,14 +317,20 @@ void sssp_step(suminc_ctx* c, uint32_t* frontier_out) {
 
 void sssp_download(suminc_ctx* c, uint32_t* dist, uint32_t* parent) {
   SUMINC_REQUIRE(c->sssp_ready, SUMINC_E_STATE, "SSSP state not initialised");
-  DevBuf dd, pp;
-  dd.ensure((size_t)c->n * 4);
-  pp.ensure((size_t)c->n * 4);
-  k_sssp_unpack<<<grid_for(c->n), kBlock, 0, c->stream>>>(c->n, c->sssp_dp.as<unsigned long long>(), c->sssp_app,
-                                                        dd.as<uint32_t>(), pp.as<uint32_t>());
-  SUMINC_HIP(hipGetLastError());
-  if (dist) SUMINC_HIP(hipMemcpyAsync(dist, dd.p, (size_t)c->n * 4, hipMemcpyDeviceToHost, c->stream));
-  if (parent) SUMINC_HIP(hipMemcpyAsync(parent, pp.p, (size_t)c->n * 4, hipMemcpyDeviceToHost, c->stream));
+  auto unpack = [c](int part, uint64_t first, uint64_t count, void* out) {
+    k_sssp_unpack<<<grid_for(count), kBlock, 0, c->stream>>>(
+        (uint32_t)count, c->sssp_dp.as<unsigned long long>() + first, c->sssp_app, part, reinterpret_cast<uint32_t*>(out));
+  };
+  uint32_t* to[2] = {dist, parent};
+  if (readback(c, {{dist, c->n, 4}, {parent, c->n, 4}}, unpack)) return;
+  DevBuf tmp;
+  tmp.ensure((size_t)c->n * 4);
+  for (int k = 0; k < 2; ++k) {
+    if (!to[k]) continue;
+    unpack(k, 0, c->n, tmp.p);
+    SUMINC_HIP(hipGetLastError());
+    SUMINC_HIP(hipMemcpyAsync(to[k], tmp.p, (size_t)c->n * 4, hipMemcpyDeviceToHost, c->stream));
+  }
   SUMINC_HIP(hipStreamSynchronize(c->stream));
 }
 

@@ -24,6 +24,7 @@
 #include "device.hpp"
 #include "extrap.hpp"
 #include "pr.hpp"
+#include "readback.hpp"
 
 namespace suminc {
 
@@ -819,6 +820,12 @@ __global__ void __launch_bounds__(kBlock) k_php_coef_csr(uint32_t n, const uint3
   }
 }
 
+__global__ void __launch_bounds__(kBlock) k_copy_f64(uint32_t n, const double* __restrict__ src,
+                                                     double* __restrict__ dst) {
+  const uint32_t v = blockIdx.x * kBlock + threadIdx.x;
+  if (v < n) dst[v] = src[v];
+}
+
 __global__ void k_php_seed(uint32_t n, uint32_t src, float* __restrict__ p) {
   const uint32_t v = blockIdx.x * blockDim.x + threadIdx.x;
   if (v < n) p[v] = v == src ? 1.f : 0.f;
@@ -848,6 +855,11 @@ static void php_run_t(suminc_ctx* c, uint32_t src, double d, double* values, sum
   const uint32_t* pos = S.in.compact ? S.in.pos.as<uint32_t>() : nullptr;
   wpr_series<T>(c, series_state<T>(c, S, pos != nullptr), R, &S.bin_in, pos, S.php_a_in.as<T>(),
                 seed.as<float>(), (T)1, c->prm.termcheck_threshold, false, nullptr, S.php64.as<double>(), st);
+  if (readback(c, {{values, n, 8}}, [c, &S](int, uint64_t first, uint64_t count, void* out) {
+        k_copy_f64<<<grid_for(count), kBlock, 0, c->stream>>>((uint32_t)count, S.php64.as<double>() + first,
+                                                             reinterpret_cast<double*>(out));
+      }))
+    return;
   if (values) SUMINC_HIP(hipMemcpyAsync(values, S.php64.p, (size_t)n * 8, hipMemcpyDefault, c->stream));
   SUMINC_HIP(hipStreamSynchronize(c->stream));
 }
