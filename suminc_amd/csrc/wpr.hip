@@ -317,43 +317,208 @@ __global__ void k_wpr_finish(uint32_t n, const T* __restrict__ x, const T* __res
 // grid of one wave per row would pass 2^32 threads at 2^26 rows).
 constexpr unsigned kWaveGrid = 65536;
 
-// ---- weights: row sums and the per-edge coefficients of both directions ---------
-__global__ void __launch_bounds__(kBlock) k_wpr_rowsum(uint32_t n, const uint32_t* __restrict__ off,
-                                                       const float* __restrict__ w, double* __restrict__ s) {
-  const uint32_t waves = gridDim.x * (kBlock / 64);
-  for (uint32_t v = blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6); v < n; v += waves) {  // whole waves
-    double acc = 0;
-    for (uint32_t e = off[v] + lane_id(); e < off[v + 1]; e += 64) acc += (double)w[e];
+// ---- per-edge passes over the out-CSR --------------------------------------------
+// Half of R-MAT's rows are empty and most of the others short, so a wave a row left
+// most lanes idle (2^22 vertices, 50M edges: row sums 1.55 ms, coefficients 1.81 ms,
+// gradients 4.04 ms, each against about 0.1 ms for the bytes).  Sums over rows take the
+// row classes with 8 lanes a short row (k_row_sum: 0.17 ms); passes that only need to
+// know an edge's row take tiles of consecutive edges whatever the rows
+// (for_tile_edges: coefficients 0.19 ms, gradients 0.41 ms, bound by the gather of
+// lambda).
+
+// Per-edge terms of the row sums.
+struct TermWeight {  // w_uv
+  const float* w;
+  __device__ double operator()(uint32_t e) const { return (double)w[e]; }
+};
+struct TermPhp {  // w_uv, edges into the source left out; integer, float or unit weights
+  const uint32_t* col;
+  const uint32_t* wu;
+  const float* wf;
+  uint32_t src;
+  __device__ double operator()(uint32_t e) const {
+    return col[e] == src ? 0.0 : wu ? (double)wu[e] : wf ? (double)wf[e] : 1.0;
+  }
+};
+struct TermDot {  // w_uv x_v
+  const float* w;
+  const uint32_t* col;
+  const double* x;
+  __device__ double operator()(uint32_t e) const { return (double)w[e] * x[col[e]]; }
+};
+
+// out[v] = FP64 sum of f over the edges of row v, the rows with edges (a row of more
+// than kHeavyDeg: its chunks' sums in part, k_row_sum_heavy adds them), in a fixed order.
+// Workgroups as k_spmv's.
+template <class F>
+__global__ void __launch_bounds__(kBlock) k_row_sum(RowLists L, F f, double* __restrict__ out,
+                                                    double* __restrict__ part, uint32_t gh, uint32_t gw) {
+  __shared__ double s_red[kBlock / 64];
+  const uint32_t bid = blockIdx.x;
+  if (bid < gh) {
+    for (uint64_t h = bid; h < L.n_heavy; h += gh) {
+      const uint2 ch = L.heavy[h];
+      const uint32_t b = L.off[ch.x] + ch.y * kChunk;
+      const uint32_t e = min(L.off[ch.x + 1], b + kChunk);
+      double acc = 0;
+      for (uint32_t k = b + threadIdx.x; k < e; k += kBlock) acc += f(k);
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) acc += __shfl_xor(acc, o);
-    if (lane_id() == 0) s[v] = acc;
+      for (int o = 32; o > 0; o >>= 1) acc += __shfl_xor(acc, o);
+      if (lane_id() == 0) s_red[threadIdx.x >> 6] = acc;
+      __syncthreads();
+      if (threadIdx.x == 0) {
+        double t = 0;
+        for (int w = 0; w < kBlock / 64; ++w) t += s_red[w];
+        part[h] = t;
+      }
+      __syncthreads();
+    }
+    return;
+  }
+  const bool wave = bid < gh + gw;
+  const uint32_t lanes = wave ? 64u : 8u;
+  const uint32_t groups = (wave ? gw : gridDim.x - gh - gw) * (kBlock / lanes);
+  const uint32_t first = (bid - gh - (wave ? 0u : gw)) * (kBlock / lanes) + threadIdx.x / lanes;
+  const uint32_t count = wave ? L.n_wave : L.n_short;
+  const uint32_t* list = wave ? L.wave : L.shrt;
+  const uint32_t lane = threadIdx.x & (lanes - 1);
+  // whole waves: the shuffles below need every lane of a group
+  for (uint32_t i = first; i - threadIdx.x / lanes % (64 / lanes) < count; i += groups) {
+    double acc = 0;
+    const uint32_t v = i < count ? list[i] : 0u;
+    if (i < count) {
+      const uint32_t e = L.off[v + 1];
+      for (uint32_t k = L.off[v] + lane; k < e; k += lanes) acc += f(k);
+    }
+    for (uint32_t o = lanes >> 1; o > 0; o >>= 1) acc += __shfl_xor(acc, o);
+    if (lane == 0 && i < count) out[v] = acc;
   }
 }
 
-// a_e = d w_e / s_src for the out-CSR (edge-parallel over rows via the tile rows)
-template <class T>
-__global__ void __launch_bounds__(kBlock) k_wpr_coef_csr(uint32_t n, const uint32_t* __restrict__ off,
-                                                         const float* __restrict__ w, const double* __restrict__ s,
-                                                         double d, T* __restrict__ a) {
-  const uint32_t waves = gridDim.x * (kBlock / 64);
-  for (uint32_t v = blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6); v < n; v += waves) {
-    const double inv = s[v] > 0 ? d / s[v] : 0.0;
-    for (uint32_t e = off[v] + lane_id(); e < off[v + 1]; e += 64) a[e] = (T)((double)w[e] * inv);
+// One wave per row of more than kHeavyDeg edges (the entries of chunk 0; a row's
+// chunks follow each other): its chunk sums added up.
+__global__ void __launch_bounds__(kBlock) k_row_sum_heavy(RowLists L, const double* __restrict__ part,
+                                                          double* __restrict__ out) {
+  const uint64_t h = (uint64_t)blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6);
+  if (h >= L.n_heavy) return;
+  const uint2 ch = L.heavy[h];
+  if (ch.y != 0) return;
+  const uint32_t nch = (L.off[ch.x + 1] - L.off[ch.x] + kChunk - 1) / kChunk;
+  double acc = 0;
+  for (uint32_t k = lane_id(); k < nch; k += 64) acc += part[h + k];
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) acc += __shfl_xor(acc, o);
+  if (lane_id() == 0) out[ch.x] = acc;
+}
+
+// A tile of kTileE consecutive edges of a CSR per workgroup; tile_row[t] is the row of
+// edge t * kTileE (tile_row[tiles]: the last row), made once per graph.
+constexpr uint32_t kTileE = 2048;
+
+__global__ void k_tile_rows(const uint32_t* __restrict__ off, uint32_t n, uint64_t m, uint32_t tiles,
+                            uint32_t* __restrict__ tile_row) {
+  const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t > tiles) return;
+  if (t == tiles) {
+    tile_row[t] = n - 1;
+    return;
+  }
+  const uint32_t e = t * kTileE;
+  uint32_t lo = 0, hi = n - 1;  // the last row that starts at or before e is the row of e
+  while (lo < hi) {
+    const uint32_t mid = lo + (hi - lo + 1) / 2;
+    if (off[mid] <= e) lo = mid; else hi = mid - 1;
+  }
+  tile_row[t] = lo;
+}
+
+// fn(edge, row) for the edges of the workgroup's tile, consecutive threads taking
+// consecutive edges.  Every row that starts inside the tile marks its first edge; a
+// running maximum over the tile gives each edge its row.
+template <class Fn>
+__device__ __forceinline__ void for_tile_edges(const uint32_t* __restrict__ off, uint64_t m,
+                                               const uint32_t* __restrict__ tile_row, Fn&& fn) {
+  constexpr int kPer = kTileE / kBlock;
+  __shared__ uint32_t s_row[kTileE];
+  __shared__ uint32_t s_w[kBlock / 64];
+  const uint32_t t = blockIdx.x;
+  const uint64_t e0 = (uint64_t)t * kTileE;
+  const uint32_t ne = (uint32_t)(m - e0 < kTileE ? m - e0 : kTileE);
+  const uint32_t r0 = tile_row[t], r1 = tile_row[t + 1];
+  if (r1 - r0 > 32 * kTileE) {  // mostly empty rows: a search per edge passes over fewer of them
+    for (uint32_t i = threadIdx.x; i < ne; i += kBlock) {
+      const uint32_t e = (uint32_t)e0 + i;
+      uint32_t lo = r0, hi = r1;
+      while (lo < hi) {
+        const uint32_t mid = lo + (hi - lo + 1) / 2;
+        if (off[mid] <= e) lo = mid; else hi = mid - 1;
+      }
+      fn(e, lo);
+    }
+    return;
+  }
+#pragma unroll
+  for (int j = 0; j < kPer; ++j) s_row[j * kBlock + threadIdx.x] = 0;
+  __syncthreads();
+  for (uint32_t r = r0 + 1 + threadIdx.x; r <= r1; r += kBlock) {
+    const uint32_t b = off[r], e = off[r + 1];
+    if (e > b && b - e0 < ne) s_row[b - (uint32_t)e0] = r - r0;
+  }
+  __syncthreads();
+  uint32_t x[kPer], run = 0;
+#pragma unroll
+  for (int j = 0; j < kPer; ++j) {
+    run = max(run, s_row[threadIdx.x * kPer + j]);
+    x[j] = run;
+  }
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const uint32_t y = __shfl_up(run, o);
+    if (lane_id() >= o) run = max(run, y);
+  }
+  if (lane_id() == 63) s_w[threadIdx.x >> 6] = run;
+  uint32_t before = __shfl_up(run, 1);
+  if (lane_id() == 0) before = 0;
+  __syncthreads();
+  for (uint32_t w = 0; w < threadIdx.x >> 6; ++w) before = max(before, s_w[w]);
+#pragma unroll
+  for (int j = 0; j < kPer; ++j) s_row[threadIdx.x * kPer + j] = max(before, x[j]);
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < kPer; ++j) {
+    const uint32_t i = j * kBlock + threadIdx.x;
+    if (i < ne) fn((uint32_t)e0 + i, r0 + s_row[i]);
   }
 }
 
-// the in-CSR copy: a_csc[i] = a_csr[eid[i]]
-template <class T>
-__global__ void k_wpr_gather(uint64_t m, const uint32_t* __restrict__ eid, const T* __restrict__ src,
-                             T* __restrict__ dst) {
-  const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < m) dst[i] = src[eid[i]];
+// a_e = d f(e) / s_row
+template <class T, class F>
+__global__ void __launch_bounds__(kBlock) k_wpr_coef(const uint32_t* __restrict__ off, uint64_t m,
+                                                     const uint32_t* __restrict__ tile_row, F f,
+                                                     const double* __restrict__ s, double d, T* __restrict__ a) {
+  for_tile_edges(off, m, tile_row, [&](uint32_t e, uint32_t v) {
+    const double sv = s[v];
+    const double inv = sv > 0 ? d / sv : 0.0;
+    a[e] = (T)(f(e) * inv);
+  });
 }
 
-__global__ void k_wpr_gather_f(uint64_t m, const uint32_t* __restrict__ eid, const float* __restrict__ src,
-                               uint32_t* __restrict__ dst) {
-  const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < m) dst[i] = __float_as_uint(src[eid[i]]);
+// dst[i] = src[eid[i]]: the coefficients in CSC or layout order.  kGatherPer values a
+// thread, their loads in flight together.
+constexpr int kGatherPer = 4;
+template <class T>
+__global__ void __launch_bounds__(kBlock) k_wpr_gather(uint64_t m, const uint32_t* __restrict__ eid,
+                                                       const T* __restrict__ src, T* __restrict__ dst) {
+  const uint64_t base = (uint64_t)blockIdx.x * (kBlock * kGatherPer) + threadIdx.x;
+  uint32_t e[kGatherPer];
+#pragma unroll
+  for (int j = 0; j < kGatherPer; ++j) e[j] = base + j * kBlock < m ? __builtin_nontemporal_load(eid + base + j * kBlock) : 0u;
+  T x[kGatherPer];
+#pragma unroll
+  for (int j = 0; j < kGatherPer; ++j) x[j] = src[e[j]];
+#pragma unroll
+  for (int j = 0; j < kGatherPer; ++j)
+    if (base + j * kBlock < m) __builtin_nontemporal_store(x[j], dst + base + j * kBlock);
 }
 
 // CSR edge id of every CSC position: sort (dst, src) keys with the edge index
@@ -371,43 +536,39 @@ __global__ void k_wpr_edge_keys(const uint32_t* __restrict__ off, uint32_t n, ui
 
 // ---- gradients -------------------------------------------------------------------
 // grad_w[e] for CSR edge e = (u -> v): (d r_u / s_u) lambda_v - (r_u / s_u) y_u with
-// y_u = sum_k a_uk lambda_k = d sum_k W[u,k] lambda_k.  One wave per row.
-__global__ void __launch_bounds__(kBlock) k_wpr_grad_w(uint32_t n, const uint32_t* __restrict__ off,
-                                                       const uint32_t* __restrict__ col, const double* __restrict__ s,
-                                                       const double* __restrict__ r, const double* __restrict__ lam,
-                                                       const double* __restrict__ yl, double d,
-                                                       float* __restrict__ g32, double* __restrict__ g64) {
-  const uint32_t waves = gridDim.x * (kBlock / 64);
-  for (uint32_t u = blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6); u < n; u += waves) {
-    const double ru = s[u] > 0 ? r[u] / s[u] : 0.0;  // a row without weight mass has no gradient
-    const double sub = ru * yl[u];
-    for (uint32_t e = off[u] + lane_id(); e < off[u + 1]; e += 64) {
-      const double g = d * ru * lam[col[e]] - sub;
-      if (g32) g32[e] = (float)g;
-      if (g64) g64[e] = g;
-    }
-  }
+// y_u = sum_k a_uk lambda_k = (d / s_u) sum_k w_uk lambda_k.  rows: per vertex
+// (d r_u / s_u, r_u y_u / s_u).
+__global__ void __launch_bounds__(kBlock) k_wpr_grad_rows(uint32_t n, const double* __restrict__ s,
+                                                          const double* __restrict__ r,
+                                                          const double* __restrict__ dot, double d,
+                                                          double2* __restrict__ rows) {
+  const uint32_t u = blockIdx.x * kBlock + threadIdx.x;
+  if (u >= n) return;
+  const double su = s[u];
+  const double ru = su > 0 ? r[u] / su : 0.0;  // a row without weight mass has no gradient
+  rows[u] = make_double2(d * ru, su > 0 ? ru * (d * dot[u] / su) : 0.0);
 }
 
-__global__ void k_wpr_grad_p(uint32_t n, const double* __restrict__ lam, double d, float* __restrict__ g32,
-                             double* __restrict__ g64) {
-  const uint32_t v = blockIdx.x * blockDim.x + threadIdx.x;
-  if (v >= n) return;
-  const double g = (1.0 - d) * lam[v];
-  if (g32) g32[v] = (float)g;
-  if (g64) g64[v] = g;
+__global__ void __launch_bounds__(kBlock) k_wpr_grad_w(const uint32_t* __restrict__ off,
+                                                       const uint32_t* __restrict__ col, uint64_t m,
+                                                       const uint32_t* __restrict__ tile_row,
+                                                       const double2* __restrict__ rows,
+                                                       const double* __restrict__ lam, float* __restrict__ g) {
+  for_tile_edges(off, m, tile_row, [&](uint32_t e, uint32_t u) {
+    const double2 x = rows[u];
+    g[e] = (float)(x.x * lam[col[e]] - x.y);
+  });
 }
 
-template <class T>
-__global__ void k_to_t(uint32_t n, const double* __restrict__ src, T* __restrict__ dst) {
+__global__ void k_wpr_grad_p(uint32_t n, const double* __restrict__ lam, double d, float* __restrict__ g) {
   const uint32_t v = blockIdx.x * blockDim.x + threadIdx.x;
-  if (v < n) dst[v] = (T)src[v];
+  if (v < n) g[v] = (float)((1.0 - d) * lam[v]);
 }
 
-template <class T>
-__global__ void k_to_f64(uint32_t n, const T* __restrict__ src, double* __restrict__ dst) {
-  const uint32_t v = blockIdx.x * blockDim.x + threadIdx.x;
-  if (v < n) dst[v] = (double)src[v];
+// the layout's edges as indices of the CSR: eid[i] <- csr_of[eid[i]]
+__global__ void k_wpr_compose(uint64_t m, const uint32_t* __restrict__ csr_of, uint32_t* __restrict__ eid) {
+  const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < m) eid[i] = csr_of[eid[i]];
 }
 
 // ---------------------------------------------------------------------------------
@@ -450,13 +611,18 @@ struct WprState {
   uint64_t fwd_coef_version = ~0ull;
   WprDir out, in;
   DevBuf eid;                        // CSR edge id per CSC position
+  DevBuf tile_row;                   // the row of the first edge of every edge tile of the CSR
+  DevBuf row_part;                   // chunk sums of the long rows
   DevBuf s;                          // row sums (f64)
+  DevBuf in_f, out_f, grad_w;        // FP32 vectors in and out of host or foreign memory
+  DevBuf dot, grad_rows;             // sum_k w_uk lambda_k; the gradient's two terms per row
   DevBuf a_out, a_in;                // coefficients d w / s (T) in CSR / CSC order
   DevBuf x, y, sum, comp;            // round state (T)
   DevBuf xc;                         // x at the compact positions (large graphs)
-  DevBuf r64, lam64, yl64;           // FP64 results of the last forward / backward
+  DevBuf r64, lam64;                 // FP64 results of the last forward / backward
   DevBuf l1;                         // sum |seed|
   DevBuf php_a_out, php_a_in, php64;  // PHP: coefficients (T) in CSR / CSC order, FP64 result
+  DevBuf php_s;                      // PHP: row sums (f64)
   // binned series rounds (large graphs, the PageRank pull's rule): the forward over
   // the CSC, the adjoint over the CSR, their coefficients in layout order; built for
   // elements of bin_es bytes
@@ -527,29 +693,18 @@ static void wpr_prepare_graph(suminc_ctx* c, WprState& S) {
                      S.out.compact ? S.out.colc.as<uint32_t>() : c->out_col.as<uint32_t>(), src_out, es, win,
                      c->prm.pull_bin_direct, m, true);
   }
+  if (S.bin_in.n_parts)  // its coefficients come from the CSR order directly
+    k_wpr_compose<<<grid_for(m), kBlock, 0, c->stream>>>(m, S.eid.as<uint32_t>(), S.bin_in.eid.as<uint32_t>());
+  const uint32_t tiles = (uint32_t)((m + kTileE - 1) / kTileE);
+  S.tile_row.ensure((size_t)tiles * 4 + 4);
+  k_tile_rows<<<grid_for((uint64_t)tiles + 1), kBlock, 0, c->stream>>>(c->out_off.as<uint32_t>(), n, m, tiles,
+                                                                      S.tile_row.as<uint32_t>());
+  SUMINC_HIP(hipGetLastError());
+  S.row_part.ensure(S.out.n_heavy * 8 + 8);
   S.bin_es = es;
   S.graph_version = c->graph_version;
   S.coef_version = ~0ull;
   S.fwd_ready = false;
-}
-
-template <class T>
-static void wpr_prepare_coef(suminc_ctx* c, WprState& S) {
-  const int prec = sizeof(T) == 8 ? SUMINC_PR_FP64 : SUMINC_PR_FP32_KAHAN;
-  if (S.coef_version == S.weights_version && S.coef_prec == prec) return;
-  const uint32_t n = c->n;
-  const uint64_t m = c->m;
-  S.s.ensure((size_t)n * 8 + 8);
-  S.a_out.ensure(m * sizeof(T) + 8);
-  S.a_in.ensure(m * sizeof(T) + 8);
-  const unsigned gw = grid_for(n, kBlock / 64, kWaveGrid);
-  k_wpr_rowsum<<<gw, kBlock, 0, c->stream>>>(n, c->out_off.as<uint32_t>(), c->out_w.as<float>(), S.s.as<double>());
-  k_wpr_coef_csr<T><<<gw, kBlock, 0, c->stream>>>(n, c->out_off.as<uint32_t>(), c->out_w.as<float>(),
-                                                  S.s.as<double>(), c->prm.damping, S.a_out.as<T>());
-  if (m) k_wpr_gather<T><<<grid_for(m), kBlock, 0, c->stream>>>(m, S.eid.as<uint32_t>(), S.a_out.as<T>(), S.a_in.as<T>());
-  SUMINC_HIP(hipGetLastError());
-  S.coef_version = S.weights_version;
-  S.coef_prec = prec;
 }
 
 // compact: the renamed columns when the direction has them (then the gathered
@@ -573,6 +728,50 @@ static void spmv(suminc_ctx* c, const RowLists& R, const T* a, const T* x, T* y,
   const uint32_t gw = R.n_wave ? grid_for(R.n_wave, kBlock / 64, 8192) : 0u;
   const uint32_t gs = R.n_short ? grid_for(R.n_short, kBlock, 8192) : 0u;
   if (gh + gw + gs) k_spmv<T><<<gh + gw + gs, kBlock, 0, c->stream>>>(R, a, x, y, cnt, gh, gw);
+}
+
+// out = per row FP64 sums of f over the out-edges (0 for empty rows).
+template <class F>
+static void row_sum(suminc_ctx* c, WprState& S, F f, double* out) {
+  const RowLists R = lists_of(S.out, c->out_off, c->out_col, false);
+  SUMINC_HIP(hipMemsetAsync(out, 0, (size_t)c->n * 8, c->stream));
+  const uint32_t gh = (uint32_t)std::min<uint64_t>(R.n_heavy, 8192);
+  const uint32_t gw = R.n_wave ? grid_for(R.n_wave, kBlock / 64, 8192) : 0u;
+  const uint32_t gs = R.n_short ? grid_for(R.n_short, kBlock / 8, 16384) : 0u;
+  if (gh + gw + gs)
+    k_row_sum<F><<<gh + gw + gs, kBlock, 0, c->stream>>>(R, f, out, S.row_part.as<double>(), gh, gw);
+  if (R.n_heavy)
+    k_row_sum_heavy<<<grid_for(R.n_heavy, kBlock / 64), kBlock, 0, c->stream>>>(R, S.row_part.as<double>(), out);
+  SUMINC_HIP(hipGetLastError());
+}
+
+// a = d f / s in CSR order, and in CSC order for the row classes (the binned rounds
+// take theirs from the CSR order).
+template <class T, class F>
+static void edge_coefs(suminc_ctx* c, WprState& S, F f, const double* s, double d, T* a_out, DevBuf& a_in) {
+  const uint64_t m = c->m;
+  if (!m) return;
+  k_wpr_coef<T, F><<<(unsigned)((m + kTileE - 1) / kTileE), kBlock, 0, c->stream>>>(
+      c->out_off.as<uint32_t>(), m, S.tile_row.as<uint32_t>(), f, s, d, a_out);
+  if (!S.bin_in.n_parts) {
+    a_in.ensure(m * sizeof(T) + 8);
+    k_wpr_gather<T><<<grid_for(m, kBlock * kGatherPer), kBlock, 0, c->stream>>>(m, S.eid.as<uint32_t>(), a_out,
+                                                                              a_in.as<T>());
+  }
+  SUMINC_HIP(hipGetLastError());
+}
+
+template <class T>
+static void wpr_prepare_coef(suminc_ctx* c, WprState& S) {
+  const int prec = sizeof(T) == 8 ? SUMINC_PR_FP64 : SUMINC_PR_FP32_KAHAN;
+  if (S.coef_version == S.weights_version && S.coef_prec == prec) return;
+  S.s.ensure((size_t)c->n * 8 + 8);
+  S.a_out.ensure(c->m * sizeof(T) + 8);
+  const TermWeight w{c->out_w.as<float>()};
+  row_sum(c, S, w, S.s.as<double>());
+  edge_coefs<T>(c, S, w, S.s.as<double>(), c->prm.damping, S.a_out.as<T>(), S.a_in);
+  S.coef_version = S.weights_version;
+  S.coef_prec = prec;
 }
 
 // Device buffers of one series run: the round state (x, y, the compensated sum),
@@ -635,19 +834,21 @@ static SeriesBufs<T> series_state(suminc_ctx* c, WprState& S, bool compact) {
 }
 
 // Runs sum = sum_t x_t with x_{t+1} = A x_t from x_0 = scale * seed until
-// sum|x| < tol.  Result (FP64) in out64, optionally FP32 in out32 (either may be
+// sum|x| < tol.  A's coefficients: a in the order of R's rows, a_csr in the CSR's (the
+// binned rounds).  Result (FP64) in out64, optionally FP32 in out32 (either may be
 // null).  pos != nullptr: R's columns are compact positions, and the rounds
 // gather the compact copy of x (B.xc).  Allocates nothing itself.
 template <class T>
 static void wpr_series(suminc_ctx* c, const SeriesBufs<T>& B, const RowLists& R, const BinLayout* L,
-                       const uint32_t* pos, const T* a, const float* seed_dev, T scale, double tol_abs, bool relative,
+                       const uint32_t* pos, const T* a, const T* a_csr, const float* seed_dev, T scale, double tol_abs, bool relative,
                        float* out32, double* out64, suminc_stats* st) {
   const uint32_t n = c->n;
-  // the binned layout of R's direction when it exists: its coefficients taken from a
-  // in layout order, the rounds through the gather and summing passes
+  // the binned layout of R's direction when it exists: its coefficients taken in layout
+  // order, the rounds through the gather and summing passes
   const bool binned = L && L->n_parts;
   if (binned && L->m)
-    k_wpr_gather<T><<<grid_for(L->m), kBlock, 0, c->stream>>>(L->m, L->eid.as<uint32_t>(), a, L->coef.as<T>());
+    k_wpr_gather<T><<<grid_for(L->m, kBlock * kGatherPer), kBlock, 0, c->stream>>>(L->m, L->eid.as<uint32_t>(), a_csr,
+                                                                                  L->coef.as<T>());
   T* xc = pos ? B.xc : nullptr;
   const unsigned g = grid_for(n);
   const unsigned gs = grid_for(n, kBlock * kStepPer);  // the round's vertex pass and its partials
@@ -704,13 +905,52 @@ void wpr_set_weights(suminc_ctx* c, const float* w) {
   if (c->m) {
     SUMINC_HIP(hipMemcpyAsync(c->out_w.p, w, c->m * 4, hipMemcpyDefault, c->stream));
     wpr_prepare_graph(c, S);
-    k_wpr_gather_f<<<grid_for(c->m), kBlock, 0, c->stream>>>(c->m, S.eid.as<uint32_t>(), c->out_w.as<float>(),
-                                                             c->in_w.as<uint32_t>());
+    k_wpr_gather<float><<<grid_for(c->m, kBlock * kGatherPer), kBlock, 0, c->stream>>>(
+        c->m, S.eid.as<uint32_t>(), c->out_w.as<float>(), c->in_w.as<float>());
     SUMINC_HIP(hipGetLastError());
     SUMINC_HIP(hipStreamSynchronize(c->stream));
   }
   S.weights_version++;
   S.fwd_ready = false;
+}
+
+// Device memory of the context's GPU, which a kernel can be handed as it is.
+static bool own_device(const suminc_ctx* c, const void* p) {
+  hipPointerAttribute_t a{};
+  if (hipPointerGetAttributes(&a, p) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  return a.type == hipMemoryTypeDevice && a.device == c->device;
+}
+
+// A caller's vector as kernels read it: itself, or its copy in buf.
+static const float* vector_in(suminc_ctx* c, const float* p, uint64_t count, DevBuf& buf) {
+  if (own_device(c, p)) return p;
+  buf.ensure(count * 4 + 4);
+  SUMINC_HIP(hipMemcpyAsync(buf.p, p, count * 4, hipMemcpyDefault, c->stream));
+  return buf.as<float>();
+}
+
+// Where kernels write a result of the caller's (null: nowhere to bring it), and its way
+// there afterwards.
+static float* vector_out(suminc_ctx* c, float* p, uint64_t count, DevBuf& buf) {
+  if (p && own_device(c, p)) return p;
+  buf.ensure(count * 4 + 4);
+  return buf.as<float>();
+}
+__global__ void __launch_bounds__(kBlock) k_copy_f32(uint32_t n, const float* __restrict__ src,
+                                                     float* __restrict__ dst) {
+  const uint32_t v = blockIdx.x * kBlock + threadIdx.x;
+  if (v < n) dst[v] = src[v];
+}
+static void vector_home(suminc_ctx* c, float* p, const float* dev, uint64_t count) {
+  if (!p || p == dev || !count) return;
+  if (readback(c, {{p, count, 4}}, [c, dev](int, uint64_t first, uint64_t k, void* out) {
+        k_copy_f32<<<grid_for(k), kBlock, 0, c->stream>>>((uint32_t)k, dev + first, reinterpret_cast<float*>(out));
+      }))
+    return;
+  SUMINC_HIP(hipMemcpyAsync(p, dev, count * 4, hipMemcpyDefault, c->stream));
 }
 
 template <class T>
@@ -719,17 +959,14 @@ static void wpr_forward_t(suminc_ctx* c, const float* p, float* r, suminc_stats*
   wpr_prepare_graph(c, S);
   wpr_prepare_coef<T>(c, S);
   const uint32_t n = c->n;
-  DevBuf pd, r32;
-  pd.ensure((size_t)n * 4);
-  SUMINC_HIP(hipMemcpyAsync(pd.p, p, (size_t)n * 4, hipMemcpyDefault, c->stream));
+  const float* pd = vector_in(c, p, n, S.in_f);
   S.r64.ensure((size_t)n * 8 + 8);
-  r32.ensure((size_t)n * 4 + 4);
+  float* rd = r ? vector_out(c, r, n, S.out_f) : nullptr;
   const RowLists R = lists_of(S.in, c->in_off, c->in_col, true);
   const uint32_t* pos = S.in.compact ? S.in.pos.as<uint32_t>() : nullptr;
-  wpr_series<T>(c, series_state<T>(c, S, pos != nullptr), R, &S.bin_in, pos, S.a_in.as<T>(), pd.as<float>(),
-                (T)(1.0 - c->prm.damping), c->prm.termcheck_threshold,
-                false, r32.as<float>(), S.r64.as<double>(), st);
-  if (r) SUMINC_HIP(hipMemcpyAsync(r, r32.p, (size_t)n * 4, hipMemcpyDefault, c->stream));
+  wpr_series<T>(c, series_state<T>(c, S, pos != nullptr), R, &S.bin_in, pos, S.a_in.as<T>(), S.a_out.as<T>(), pd,
+                (T)(1.0 - c->prm.damping), c->prm.termcheck_threshold, false, rd, S.r64.as<double>(), st);
+  vector_home(c, r, rd, n);
   SUMINC_HIP(hipStreamSynchronize(c->stream));
   S.fwd_ready = true;
   S.fwd_coef_version = S.weights_version;
@@ -743,37 +980,34 @@ static void wpr_backward_t(suminc_ctx* c, const float* cvec, float* grad_p, floa
   wpr_prepare_coef<T>(c, S);
   const uint32_t n = c->n;
   const uint64_t m = c->m;
-  DevBuf cd, gp32, gw32;
-  cd.ensure((size_t)n * 4);
-  SUMINC_HIP(hipMemcpyAsync(cd.p, cvec, (size_t)n * 4, hipMemcpyDefault, c->stream));
+  const double d = c->prm.damping;
+  const float* cd = vector_in(c, cvec, n, S.in_f);
   S.lam64.ensure((size_t)n * 8 + 8);
-  S.yl64.ensure((size_t)n * 8 + 8);
   const RowLists R = lists_of(S.out, c->out_off, c->out_col, true);
   const uint32_t* pos = S.out.compact ? S.out.pos.as<uint32_t>() : nullptr;
-  wpr_series<T>(c, series_state<T>(c, S, pos != nullptr), R, &S.bin_out, pos, S.a_out.as<T>(), cd.as<float>(),
-                (T)1, c->prm.termcheck_threshold, true, nullptr,
-                S.lam64.as<double>(), st);
-  // y_u = sum_k a_uk lambda_k (one more product, in FP64)
-  DevBuf lam_t, y_t;
-  lam_t.ensure((size_t)n * sizeof(T) + 8);
-  y_t.ensure((size_t)n * sizeof(T) + 8);
-  SUMINC_HIP(hipMemsetAsync(y_t.p, 0, (size_t)n * sizeof(T), c->stream));
-  k_to_t<T><<<grid_for(n), kBlock, 0, c->stream>>>(n, S.lam64.as<double>(), lam_t.as<T>());
-  spmv<T>(c, lists_of(S.out, c->out_off, c->out_col, false), S.a_out.as<T>(), lam_t.as<T>(), y_t.as<T>(), nullptr);
-  DevBuf yd;
-  yd.ensure((size_t)n * 8 + 8);
-  k_to_f64<T><<<grid_for(n), kBlock, 0, c->stream>>>(n, y_t.as<T>(), yd.as<double>());
-  SUMINC_HIP(hipGetLastError());
-  gp32.ensure((size_t)n * 4 + 4);
-  gw32.ensure(m * 4 + 4);
-  k_wpr_grad_p<<<grid_for(n), kBlock, 0, c->stream>>>(n, S.lam64.as<double>(), c->prm.damping, gp32.as<float>(),
-                                                      nullptr);
-  k_wpr_grad_w<<<grid_for(n, kBlock / 64, kWaveGrid), kBlock, 0, c->stream>>>(
-      n, c->out_off.as<uint32_t>(), c->out_col.as<uint32_t>(), S.s.as<double>(), S.r64.as<double>(),
-      S.lam64.as<double>(), yd.as<double>(), c->prm.damping, gw32.as<float>(), nullptr);
-  SUMINC_HIP(hipGetLastError());
-  if (grad_p) SUMINC_HIP(hipMemcpyAsync(grad_p, gp32.p, (size_t)n * 4, hipMemcpyDefault, c->stream));
-  if (grad_w && m) SUMINC_HIP(hipMemcpyAsync(grad_w, gw32.p, m * 4, hipMemcpyDefault, c->stream));
+  wpr_series<T>(c, series_state<T>(c, S, pos != nullptr), R, &S.bin_out, pos, S.a_out.as<T>(), S.a_out.as<T>(), cd,
+                (T)1, c->prm.termcheck_threshold, true, nullptr, S.lam64.as<double>(), st);
+  const double* lam = S.lam64.as<double>();
+  if (grad_p) {
+    float* gp = vector_out(c, grad_p, n, S.out_f);
+    k_wpr_grad_p<<<grid_for(n), kBlock, 0, c->stream>>>(n, lam, d, gp);
+    SUMINC_HIP(hipGetLastError());
+    vector_home(c, grad_p, gp, n);
+  }
+  if (grad_w && m) {
+    // one more product, in FP64 from the weights themselves
+    S.dot.ensure((size_t)n * 8 + 8);
+    S.grad_rows.ensure((size_t)n * 16 + 16);
+    row_sum(c, S, TermDot{c->out_w.as<float>(), c->out_col.as<uint32_t>(), lam}, S.dot.as<double>());
+    k_wpr_grad_rows<<<grid_for(n), kBlock, 0, c->stream>>>(n, S.s.as<double>(), S.r64.as<double>(), S.dot.as<double>(),
+                                                          d, S.grad_rows.as<double2>());
+    float* gw = vector_out(c, grad_w, m, S.grad_w);
+    k_wpr_grad_w<<<(unsigned)((m + kTileE - 1) / kTileE), kBlock, 0, c->stream>>>(
+        c->out_off.as<uint32_t>(), c->out_col.as<uint32_t>(), m, S.tile_row.as<uint32_t>(), S.grad_rows.as<double2>(),
+        lam, gw);
+    SUMINC_HIP(hipGetLastError());
+    vector_home(c, grad_w, gw, m);
+  }
   SUMINC_HIP(hipStreamSynchronize(c->stream));
 }
 
@@ -799,27 +1033,6 @@ void wpr_backward(suminc_ctx* c, const float* cvec, float* grad_p, float* grad_w
 // (frag.weight_sum, :30-45); nothing enters the source again.  That is the weighted
 // series x_{t+1} = A x_t with a_uv = d w_uv / s_u (0 into the source), x_0 = e_src,
 // value = sum_t x_t: the weighted-PageRank rounds over the same CSC row classes.
-template <class T>
-__global__ void __launch_bounds__(kBlock) k_php_coef_csr(uint32_t n, const uint32_t* __restrict__ off,
-                                                         const uint32_t* __restrict__ col,
-                                                         const uint32_t* __restrict__ wu,
-                                                         const float* __restrict__ wf, uint32_t src, double d,
-                                                         T* __restrict__ a) {
-  const uint32_t waves = gridDim.x * (kBlock / 64);
-  for (uint32_t v = blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6); v < n; v += waves) {  // whole waves
-    double acc = 0;
-    for (uint32_t e = off[v] + lane_id(); e < off[v + 1]; e += 64)
-      if (col[e] != src) acc += wu ? (double)wu[e] : wf ? (double)wf[e] : 1.0;
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) acc += __shfl_xor(acc, o);
-    const double inv = acc > 0 ? d / acc : 0.0;
-    for (uint32_t e = off[v] + lane_id(); e < off[v + 1]; e += 64) {
-      const double w = wu ? (double)wu[e] : wf ? (double)wf[e] : 1.0;
-      a[e] = col[e] != src ? (T)(w * inv) : T(0);
-    }
-  }
-}
-
 __global__ void __launch_bounds__(kBlock) k_copy_f64(uint32_t n, const double* __restrict__ src,
                                                      double* __restrict__ dst) {
   const uint32_t v = blockIdx.x * kBlock + threadIdx.x;
@@ -838,23 +1051,19 @@ static void php_run_t(suminc_ctx* c, uint32_t src, double d, double* values, sum
   const uint32_t n = c->n;
   const uint64_t m = c->m;
   S.php_a_out.ensure(m * sizeof(T) + 8);
-  S.php_a_in.ensure(m * sizeof(T) + 8);
   S.php64.ensure((size_t)n * 8 + 8);
-  const uint32_t* wu = c->wkind == SUMINC_W_U32 ? c->out_w.as<uint32_t>() : nullptr;
-  const float* wf = c->wkind == SUMINC_W_F32 ? c->out_w.as<float>() : nullptr;
-  k_php_coef_csr<T><<<grid_for(n, kBlock / 64, kWaveGrid), kBlock, 0, c->stream>>>(
-      n, c->out_off.as<uint32_t>(), c->out_col.as<uint32_t>(), wu, wf, src, d, S.php_a_out.as<T>());
-  if (m)
-    k_wpr_gather<T><<<grid_for(m), kBlock, 0, c->stream>>>(m, S.eid.as<uint32_t>(), S.php_a_out.as<T>(),
-                                                         S.php_a_in.as<T>());
-  DevBuf seed;
-  seed.ensure((size_t)n * 4 + 4);
-  k_php_seed<<<grid_for(n), kBlock, 0, c->stream>>>(n, src, seed.as<float>());
+  S.php_s.ensure((size_t)n * 8 + 8);
+  const TermPhp w{c->out_col.as<uint32_t>(), c->wkind == SUMINC_W_U32 ? c->out_w.as<uint32_t>() : nullptr,
+                  c->wkind == SUMINC_W_F32 ? c->out_w.as<float>() : nullptr, src};
+  row_sum(c, S, w, S.php_s.as<double>());
+  edge_coefs<T>(c, S, w, S.php_s.as<double>(), d, S.php_a_out.as<T>(), S.php_a_in);
+  S.in_f.ensure((size_t)n * 4 + 4);
+  k_php_seed<<<grid_for(n), kBlock, 0, c->stream>>>(n, src, S.in_f.as<float>());
   SUMINC_HIP(hipGetLastError());
   const RowLists R = lists_of(S.in, c->in_off, c->in_col, true);
   const uint32_t* pos = S.in.compact ? S.in.pos.as<uint32_t>() : nullptr;
   wpr_series<T>(c, series_state<T>(c, S, pos != nullptr), R, &S.bin_in, pos, S.php_a_in.as<T>(),
-                seed.as<float>(), (T)1, c->prm.termcheck_threshold, false, nullptr, S.php64.as<double>(), st);
+                S.php_a_out.as<T>(), S.in_f.as<float>(), (T)1, c->prm.termcheck_threshold, false, nullptr, S.php64.as<double>(), st);
   if (readback(c, {{values, n, 8}}, [c, &S](int, uint64_t first, uint64_t count, void* out) {
         k_copy_f64<<<grid_for(count), kBlock, 0, c->stream>>>((uint32_t)count, S.php64.as<double>() + first,
                                                              reinterpret_cast<double*>(out));
@@ -929,9 +1138,8 @@ static void wpr_forward_noalloc_t(suminc_ctx* c, const float* p, float* r, sumin
   const RowLists R = lists_of(S.in, c->in_off, c->in_col, true);
   const uint32_t* pos = compact ? S.in.pos.as<uint32_t>() : nullptr;
   S.fwd_ready = false;  // the rank of this forward is not kept for a backward
-  wpr_series<T>(c, B, R, &S.bin_in, pos, S.a_in.as<T>(), p, (T)(1.0 - c->prm.damping), c->prm.termcheck_threshold,
-                false, r,
-                nullptr, st);
+  wpr_series<T>(c, B, R, &S.bin_in, pos, S.a_in.as<T>(), S.a_out.as<T>(), p, (T)(1.0 - c->prm.damping),
+                c->prm.termcheck_threshold, false, r, nullptr, st);
   SUMINC_HIP(hipStreamSynchronize(c->stream));
 }
 

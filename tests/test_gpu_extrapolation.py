@@ -196,7 +196,7 @@ def test_weighted_series_and_adjoint(gpu, prec, name):
     rng = np.random.default_rng(9)
     w = (1.0 - rng.random(len(u))).astype(np.float32)
     s = np.bincount(u, weights=w.astype(float), minlength=n)
-    M = sp.csr_matrix((DAMPING * w / s[u], (v, u)), shape=(n, n))
+    M = sp.csr_matrix((DAMPING * w.astype(float) / s[u], (v, u)), shape=(n, n))
     p = np.zeros(n, np.float32)
     p[0] = 1.0
     c = rng.standard_normal(n).astype(np.float32)

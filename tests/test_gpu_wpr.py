@@ -136,3 +136,66 @@ def test_torch_autograd(gpu):
     if "SKIP" in out.stdout:
         pytest.skip(out.stdout.strip().splitlines()[-1])
     assert out.returncode == 0 and out.stdout.strip().endswith("OK")
+
+
+@pytest.mark.parametrize("case", ["tile_edges", "long_rows", "sparse_ids", "one_edge"])
+@pytest.mark.parametrize("bin_kib", [0, 1], ids=["rows", "binned"])
+def test_edge_passes_at_their_edges(gpu, case, bin_kib):
+    """Row sums (classes of 32 and 256 edges, 2048-edge chunks), edge tiles (2048 edges,
+    rows across them, runs of empty rows on both sides of the search's limit) and layout
+    coefficients, through the gradients, against scipy's solve.  FP64 state; gradients
+    come back as FP32 (2^-24 of each; 1e-6 of the largest bounds their cancellation)."""
+    import scipy.sparse as sp
+    import scipy.sparse.linalg as sla
+
+    rng = np.random.default_rng(2)
+    if case == "tile_edges":  # row lengths around the classes, the last edge ends a tile
+        deg = np.array([0, 1, 8, 9, 31, 32, 33, 64, 255, 256, 257, 0, 0, 300, 7, 2048 - 1253 + 0], int)
+        n = 4000
+    elif case == "long_rows":
+        deg = np.array([2047, 0, 2048, 2049, 4097, 1], int)
+        n = 6000
+    elif case == "sparse_ids":  # 70,000 and 200,000 empty rows between rows of one tile
+        n = 300_000
+        deg = np.zeros(270_500, int)
+        deg[[0, 1, 70_001, 270_100, 270_499]] = [3, 5, 40, 2, 300]
+    else:
+        n, deg = 2, np.array([1], int)
+    deg = np.concatenate([deg, np.zeros(n - len(deg), int)])
+    u = np.repeat(np.arange(n), deg)
+    v = np.concatenate([np.sort(rng.choice(n - 1, k, replace=False)) for k in deg if k] or [[]]).astype(np.int64)
+    v += v >= u  # no self-loops; still increasing within a row
+    off = np.zeros(n + 1, np.uint64)
+    off[1:] = np.cumsum(deg)
+    if case == "tile_edges":
+        assert len(u) % 2048 == 0
+    w = (1.0 - rng.random(len(u))).astype(np.float32)
+    p = rng.random(n).astype(np.float32) / n
+    c = rng.standard_normal(n).astype(np.float32)
+    s = np.bincount(u, weights=w.astype(float), minlength=n)
+    M = sp.csr_matrix((DAMPING * w.astype(float) / s[u], (v, u)), shape=(n, n))
+    I = sp.eye(n, format="csc")
+    r = sla.spsolve(I - M.tocsc(), (1 - DAMPING) * p.astype(float))
+    lam = sla.spsolve(I - M.T.tocsc(), c.astype(float))
+    gw_want = (r / np.where(s > 0, s, 1))[u] * (DAMPING * lam[v] - (M.T @ lam)[u])
+    with gpu.Context(pr_precision=gpu.PR_FP64, termcheck_threshold=1e-13, max_rounds=10000,
+                     pull_bin_kib=bin_kib or -1) as ctx:
+        ctx.upload_csr(off, v.astype(np.uint32), w)
+        ctx.wpr_set_weights(w)
+        got, _ = ctx.wpr_forward(p)
+        gp, gw, _ = ctx.wpr_backward(c)
+        dev = [ctx.device_array(x) for x in (p, c, np.zeros(n, np.float32), np.zeros(n, np.float32), np.zeros_like(w))]
+        ctx.wpr_forward(dev[0], out=dev[2])
+        ctx.wpr_backward(dev[1], grad_p=dev[3], grad_w=dev[4])
+        same = [d.download() for d in dev]
+        for d in dev:
+            d.free()
+    assert np.abs(got - r).max() <= 1e-6 * np.abs(r).max()
+    assert np.abs(gp - (1 - DAMPING) * lam).max() <= 1e-6 * np.abs(lam).max()
+    # (a single edge's gradient is 0: what is left are FP64 roundings of its two terms)
+    zero = 1e-14 * (r[u] / s[u]).max() * np.abs(lam).max()
+    assert np.abs(gw - gw_want).max() <= 1e-6 * np.abs(gw_want).max() + zero
+    # into device memory directly (hub rows add in any order: a last place of FP64 before rounding)
+    for x, y in ((same[2], got), (same[3], gp), (same[4], gw)):
+        assert np.abs(x - y).max() <= 2e-7 * np.abs(y).max() + zero
+    assert np.array_equal(same[0], p) and np.array_equal(same[1], c)
