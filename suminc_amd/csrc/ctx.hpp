@@ -267,6 +267,7 @@ struct suminc_ctx {
   // batches, taken by the next query): owned by SSSP, so that PageRank and the
   // weighted PageRank, which reset the shared counters, leave pending seeds intact
   suminc::DevBuf sssp_wl0, sssp_wl1, sssp_seeds;
+  suminc::DevBuf sssp_tile;  // pull rounds: the first row of every CSC edge tile, then a count per tile
 
   // rounds enqueued before the first host check (last run's rounds + 1)
   int hint_reset = 6, hint_sssp = 8, hint_sssp_sketch = 8;
