@@ -194,8 +194,8 @@ class Context:
 
     def pr_download(self):
         n = self.graph_info()[0]
-        rank = np.zeros(n, np.float64)
-        delta = np.zeros(n, np.float64)
+        rank = np.empty(n, np.float64)
+        delta = np.empty(n, np.float64)
         self._check(self._lib.suminc_pr_download(self._h, L.ptr(rank), L.ptr(delta)))
         return rank, delta
 
@@ -391,7 +391,7 @@ class Context:
     def php_run(self, source=0, damping=float(np.float32(0.8))):
         """PHP values (FP64) from `source`; the reference's d is 0.80f."""
         n = self.graph_info()[0]
-        out = np.zeros(n)
+        out = np.empty(n)
         s = L.Stats()
         self._check(self._lib.suminc_php_run(self._h, source, float(damping), L.ptr(out), C.byref(s)))
         return out, s.as_dict()
@@ -409,8 +409,8 @@ class Context:
 
     def sssp_download(self):
         n = self.graph_info()[0]
-        dist = np.zeros(n, np.uint32)
-        parent = np.zeros(n, np.uint32)
+        dist = np.empty(n, np.uint32)
+        parent = np.empty(n, np.uint32)
         self._check(self._lib.suminc_sssp_download(self._h, L.ptr(dist), L.ptr(parent)))
         return dist, parent
 
