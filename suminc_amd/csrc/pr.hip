@@ -282,11 +282,14 @@ __global__ void __launch_bounds__(kBlock) k_pr_gather(uint32_t n, const uint32_t
   }
 }
 
-// Applies an extrapolation that was chosen by the decision that ended the run.
+// Applies an extrapolation that was chosen by the decision that ended the run (launched
+// behind every group of rounds, so that the host waits once).
 template <class T>
 __global__ void __launch_bounds__(kBlock) k_pr_extrap_end(uint32_t n, T* __restrict__ delta, const T* __restrict__ prev,
                                                           T* __restrict__ rank, float* __restrict__ comp, double eps,
-                                                          double beta) {
+                                                          const Counters* cnt) {
+  const double beta = cnt->ex.beta;
+  if (!cnt->done || !(beta > 0.0)) return;
   const uint32_t v = blockIdx.x * kBlock + threadIdx.x;
   if (v >= n) return;
   const T p = prev[v];
@@ -386,28 +389,49 @@ __device__ __forceinline__ void pull_heavy_part(uint32_t bid, uint32_t nb, T* s_
   }
 }
 
-// One launch for the three row classes: workgroups [0, gh) take the heavy chunks
-// (the longest work first), [gh, gh + gw) the wave rows, the rest the short rows,
-// so the classes' tails overlap instead of following each other.
+// The three row classes of a pull: workgroups [0, gh) take the heavy chunks (the longest
+// work first), [gh, gh + gw) the wave rows, the rest the short rows, so the classes'
+// tails overlap instead of following each other.
+struct PullRows {
+  const uint32_t* short_list;
+  const uint32_t* wave_list;
+  const uint2* chunks;
+  const unsigned long long* counts;
+  const uint32_t* ioff;
+  const uint32_t* icol;
+  uint32_t gh, gw;
+};
 template <class T>
-__global__ void __launch_bounds__(kBlock) k_pr_pull(const uint32_t* __restrict__ short_list,
-                                                    const uint32_t* __restrict__ wave_list,
-                                                    const uint2* __restrict__ chunks,
-                                                    const unsigned long long* __restrict__ counts,
-                                                    const uint32_t* __restrict__ ioff,
-                                                    const uint32_t* __restrict__ icol, const T* __restrict__ contrib,
-                                                    T* __restrict__ delta, const Counters* cnt, int gate, uint32_t gh,
-                                                    uint32_t gw) {
+__device__ __forceinline__ void pull_rows(const PullRows& p, const T* __restrict__ contrib, T* __restrict__ delta) {
   __shared__ T s_red[kBlock / 64];
-  if (!pull_runs(cnt, gate)) return;
   const uint32_t bid = blockIdx.x;
-  if (bid < gh)
-    pull_heavy_part<T>(bid, gh, s_red, chunks, counts[2], ioff, icol, contrib, delta);
-  else if (bid < gh + gw)
-    pull_wave_part<T>(bid - gh, gw, wave_list, (uint32_t)counts[1], ioff, icol, contrib, delta);
+  if (bid < p.gh)
+    pull_heavy_part<T>(bid, p.gh, s_red, p.chunks, p.counts[2], p.ioff, p.icol, contrib, delta);
+  else if (bid < p.gh + p.gw)
+    pull_wave_part<T>(bid - p.gh, p.gw, p.wave_list, (uint32_t)p.counts[1], p.ioff, p.icol, contrib, delta);
   else
-    pull_short_part<T>(bid - gh - gw, gridDim.x - gh - gw, short_list, (uint32_t)counts[0], ioff, icol, contrib,
-                       delta);
+    pull_short_part<T>(bid - p.gh - p.gw, gridDim.x - p.gh - p.gw, p.short_list, (uint32_t)p.counts[0], p.ioff, p.icol,
+                       contrib, delta);
+}
+
+template <class T>
+__global__ void __launch_bounds__(kBlock) k_pr_pull(PullRows p, const T* __restrict__ contrib, T* __restrict__ delta,
+                                                    const Counters* cnt, int gate) {
+  if (!pull_runs(cnt, gate)) return;
+  pull_rows<T>(p, contrib, delta);
+}
+
+// A plain round's scatter, push or pull as the device decided, in one launch: an empty
+// launch costs 4 us, a fifth of a round on 2^16 vertices.
+template <class T>
+__global__ void __launch_bounds__(kBlock) k_pr_scatter(PullRows p, const T* __restrict__ contrib,
+                                                       const uint32_t* __restrict__ off,
+                                                       const uint32_t* __restrict__ col, T* __restrict__ delta,
+                                                       const uint32_t* __restrict__ wl_v, const T* __restrict__ wl_c,
+                                                       const uint4* __restrict__ heavy, const Counters* cnt) {
+  if (cnt->done) return;
+  if (cnt->mode) pull_rows<T>(p, contrib, delta);
+  else pr_push_body<T, false>(off, col, delta, wl_v, wl_c, heavy, cnt, nullptr, nullptr);
 }
 
 __global__ void __launch_bounds__(1024) k_pr_end(Counters* cnt, const unsigned long long* __restrict__ act_partial,
@@ -539,14 +563,16 @@ __global__ void k_pr_from_f64(uint32_t n, T* delta, T* rank, float* comp, const 
 
 // FP64 mass balance of the state: per block of a fixed grid, the sums of
 // r + delta and of d * r over the vertices with out-edges (r = rank - comp in
-// FP32/Kahan mode); k_pr_mass_end adds the block sums in a fixed order.
+// FP32/Kahan mode); k_pr_mass_end adds the block sums in a fixed order, into
+// cnt->dpad[1] and [2].  Both return unless the run has stopped.
 constexpr unsigned kMassGrid = 1024;
 template <class T>
 __global__ void __launch_bounds__(kBlock) k_pr_mass(uint32_t n, const uint32_t* __restrict__ off,
                                                     const T* __restrict__ delta, const T* __restrict__ rank,
                                                     const float* __restrict__ comp, double d,
-                                                    double* __restrict__ partial) {
+                                                    double* __restrict__ partial, const Counters* cnt) {
   __shared__ double s_tot[kBlock / 64], s_out[kBlock / 64];
+  if (!cnt->done) return;
   double tot = 0.0, out = 0.0;
   for (uint32_t v = blockIdx.x * kBlock + threadIdx.x; v < n; v += kMassGrid * kBlock) {
     double r = (double)rank[v];
@@ -575,8 +601,9 @@ __global__ void __launch_bounds__(kBlock) k_pr_mass(uint32_t n, const uint32_t* 
   }
 }
 
-__global__ void __launch_bounds__(1024) k_pr_mass_end(const double* __restrict__ partial, double* __restrict__ out) {
+__global__ void __launch_bounds__(1024) k_pr_mass_end(const double* __restrict__ partial, Counters* cnt) {
   __shared__ double s[1024], so[1024];
+  if (!cnt->done) return;
   s[threadIdx.x] = partial[threadIdx.x];
   so[threadIdx.x] = partial[kMassGrid + threadIdx.x];
   __syncthreads();
@@ -588,8 +615,8 @@ __global__ void __launch_bounds__(1024) k_pr_mass_end(const double* __restrict__
     __syncthreads();
   }
   if (threadIdx.x == 0) {
-    out[0] = s[0];
-    out[1] = so[0];
+    cnt->dpad[1] = s[0];
+    cnt->dpad[2] = so[0];
   }
 }
 
@@ -1875,13 +1902,31 @@ void ensure_pull_heavy(suminc_ctx* c) {
   c->pull_heavy_version = c->graph_version;
 }
 
+// Workgroups for the parts of the row-class pull: as many as the largest part's items
+// (at most push_grid heavy ones, 8192 of the others).
+static PullRows pull_rows_of(suminc_ctx* c, uint32_t* grid) {
+  PullRows p;
+  p.short_list = c->pull_short.as<uint32_t>();
+  p.wave_list = c->pull_wave.as<uint32_t>();
+  p.chunks = c->pull_heavy.as<uint2>();
+  p.counts = c->pull_cnt.as<unsigned long long>();
+  p.ioff = c->in_off.as<uint32_t>();
+  p.icol = pull_cols(c);
+  p.gh = (uint32_t)std::min<uint64_t>(push_grid(), c->m / kHeavyDeg + 1);  // rows of the class, so at least its chunks / 8
+  p.gw = grid_for(c->n, kBlock / 64, (unsigned)std::min<uint64_t>(8192, c->m / kPullThread / (kBlock / 64) + 1));
+  *grid = p.gh + p.gw + grid_for(c->n, kBlock, 8192);
+  return p;
+}
+
+// Whether the pull goes by row classes (no binned, tiled or banded layout).
+static bool pull_by_rows(const suminc_ctx* c) { return !c->bins.n_parts && !c->tile_n && c->band_P <= 1; }
+
 // The pull launches of a round (kernels return unless the gate opens, see
 // pull_runs).  The list lengths stay on the device.  The contributions are at the
 // compact positions when those are in use (the columns renamed to them).
 template <class T>
 void pull_scatter(suminc_ctx* c, int gate) {
   Counters* cnt = dev_counters(c);
-  const unsigned long long* counts = c->pull_cnt.as<unsigned long long>();
   const uint32_t* icol = pull_cols(c);
   if (c->bins.n_parts) {
     bin_layout_spmv<T, false>(c, c->bins, c->pr_contrib.as<T>(), c->pr_delta.as<T>(), cnt, gate);
@@ -1911,13 +1956,9 @@ void pull_scatter(suminc_ctx* c, int gate) {
     }
     return;
   }
-  // grid: the heavy part as before (push_grid), the wave and short parts sized to
-  // the vertex count (at most 8192 workgroups each)
-  const uint32_t gh = push_grid(), gw = grid_for(c->n, kBlock / 64, 8192), gs = grid_for(c->n, kBlock, 8192);
-  k_pr_pull<T><<<gh + gw + gs, kBlock, 0, c->stream>>>(c->pull_short.as<uint32_t>(), c->pull_wave.as<uint32_t>(),
-                                                       c->pull_heavy.as<uint2>(), counts, c->in_off.as<uint32_t>(),
-                                                       icol, c->pr_contrib.as<T>(), c->pr_delta.as<T>(), cnt, gate, gh,
-                                                       gw);
+  uint32_t grid;
+  const PullRows p = pull_rows_of(c, &grid);
+  k_pr_pull<T><<<grid, kBlock, 0, c->stream>>>(p, c->pr_contrib.as<T>(), c->pr_delta.as<T>(), cnt, gate);
 }
 template void pull_scatter<float>(suminc_ctx* c, int gate);
 template void pull_scatter<double>(suminc_ctx* c, int gate);
@@ -1944,10 +1985,18 @@ static void enqueue_round(suminc_ctx* c, double eps, double T_stop, int max_roun
                                               c->wl0.as<uint32_t>(), c->wl1.as<T>(), c->heavy.as<uint4>(),
                                               c->pr_contrib.as<T>(), pull_pos(c), cnt, act);
   if (c->prof_on) SUMINC_HIP(hipEventRecord(prof_event(c, 4 * slot + 2), c->stream));
-  k_pr_push<T><<<push_grid(), kBlock, 0, c->stream>>>(c->out_off.as<uint32_t>(), c->out_col.as<uint32_t>(),
-                                                      c->pr_delta.as<T>(), c->wl0.as<uint32_t>(), c->wl1.as<T>(),
-                                                      c->heavy.as<uint4>(), cnt);
-  if (div > 0) pull_scatter<T>(c, 0);
+  if (div > 0 && pull_by_rows(c)) {
+    uint32_t grid;
+    const PullRows p = pull_rows_of(c, &grid);
+    k_pr_scatter<T><<<grid, kBlock, 0, c->stream>>>(p, c->pr_contrib.as<T>(), c->out_off.as<uint32_t>(),
+                                                    c->out_col.as<uint32_t>(), c->pr_delta.as<T>(),
+                                                    c->wl0.as<uint32_t>(), c->wl1.as<T>(), c->heavy.as<uint4>(), cnt);
+  } else {
+    k_pr_push<T><<<push_grid(), kBlock, 0, c->stream>>>(c->out_off.as<uint32_t>(), c->out_col.as<uint32_t>(),
+                                                        c->pr_delta.as<T>(), c->wl0.as<uint32_t>(), c->wl1.as<T>(),
+                                                        c->heavy.as<uint4>(), cnt);
+    if (div > 0) pull_scatter<T>(c, 0);
+  }
   if (c->prof_on) SUMINC_HIP(hipEventRecord(prof_event(c, 4 * slot + 3), c->stream));
   if (step) k_pr_end<<<1, 1024, 0, c->stream>>>(cnt, act, gc);
 }
@@ -1997,24 +2046,19 @@ static void pr_profile_rounds(suminc_ctx* c, size_t rounds) {
                  (double)n_pull * c->n * es + (double)h->push_entries * (4.0 + es);
 }
 
-// FP64 mass balance of the current state into st->mass_total / mass_defect.
-void pr_mass(suminc_ctx* c, suminc_stats* st) {
-  if (!c->pr_ready || !st) return;
-  c->mass_part.ensure((2 * kMassGrid + 2) * sizeof(double));
+// Enqueues what follows a run's last round: the extrapolation that ended it and the
+// FP64 mass balance of its state (every kernel returns unless the run has stopped).
+template <class T>
+static void enqueue_run_end(suminc_ctx* c, double eps) {
+  Counters* cnt = dev_counters(c);
+  float* comp = sizeof(T) == 4 ? c->pr_comp.as<float>() : nullptr;
+  c->mass_part.ensure(2 * kMassGrid * sizeof(double));
   double* part = c->mass_part.as<double>();
-  const double d = c->prm.damping;
-  if (c->pr_prec == SUMINC_PR_FP64)
-    k_pr_mass<double><<<kMassGrid, kBlock, 0, c->stream>>>(c->n, c->out_off.as<uint32_t>(), c->pr_delta.as<double>(),
-                                                          c->pr_rank.as<double>(), nullptr, d, part);
-  else
-    k_pr_mass<float><<<kMassGrid, kBlock, 0, c->stream>>>(c->n, c->out_off.as<uint32_t>(), c->pr_delta.as<float>(),
-                                                         c->pr_rank.as<float>(), c->pr_comp.as<float>(), d, part);
-  k_pr_mass_end<<<1, 1024, 0, c->stream>>>(part, part + 2 * kMassGrid);
-  SUMINC_HIP(hipGetLastError());
-  check_begin(c, part + 2 * kMassGrid, 2 * sizeof(double));
-  const double* h = reinterpret_cast<const double*>(check_wait(c));
-  st->mass_total = h[0];
-  st->mass_defect = h[0] - h[1] - (1.0 - d);
+  k_pr_extrap_end<T><<<grid_for(c->n), kBlock, 0, c->stream>>>(c->n, c->pr_delta.as<T>(), c->pr_prev.as<T>(),
+                                                              c->pr_rank.as<T>(), comp, eps, cnt);
+  k_pr_mass<T><<<kMassGrid, kBlock, 0, c->stream>>>(c->n, c->out_off.as<uint32_t>(), c->pr_delta.as<T>(),
+                                                   c->pr_rank.as<T>(), comp, c->prm.damping, part, cnt);
+  k_pr_mass_end<<<1, 1024, 0, c->stream>>>(part, cnt);
 }
 
 // Runs rounds until the device sets the stop flag; host polls every `group` rounds.
@@ -2035,24 +2079,14 @@ void pr_run(suminc_ctx* c, suminc_stats* st) {
       if (c->pr_prec == SUMINC_PR_FP64) enqueue_round<double>(c, eps, T, max_rounds, div, slot, false);
       else enqueue_round<float>(c, eps, T, max_rounds, div, slot, false);
     }
+    if (c->pr_prec == SUMINC_PR_FP64) enqueue_run_end<double>(c, eps);
+    else enqueue_run_end<float>(c, eps);
     SUMINC_HIP(hipGetLastError());
+    SUMINC_HIP(hipEventRecord(c->ev_stop, c->stream));
     read_counters(c);
     if (c->host_counters->done) break;
     group = slot < 20 ? 4 : std::min(32, 2 * group);
   }
-  const double beta = c->host_counters->ex.beta;
-  if (beta > 0.0) {  // chosen by the decision that ended the run
-    const unsigned g = grid_for(c->n);
-    if (c->pr_prec == SUMINC_PR_FP64)
-      k_pr_extrap_end<double><<<g, kBlock, 0, c->stream>>>(c->n, c->pr_delta.as<double>(), c->pr_prev.as<double>(),
-                                                          c->pr_rank.as<double>(), nullptr, eps, beta);
-    else
-      k_pr_extrap_end<float><<<g, kBlock, 0, c->stream>>>(c->n, c->pr_delta.as<float>(), c->pr_prev.as<float>(),
-                                                         c->pr_rank.as<float>(), c->pr_comp.as<float>(), eps, beta);
-    SUMINC_HIP(hipGetLastError());
-  }
-  SUMINC_HIP(hipEventRecord(c->ev_stop, c->stream));
-  SUMINC_HIP(hipEventSynchronize(c->ev_stop));
   float ms = 0;
   SUMINC_HIP(hipEventElapsedTime(&ms, c->ev_start, c->ev_stop));
   Counters* h = c->host_counters;
@@ -2066,7 +2100,8 @@ void pr_run(suminc_ctx* c, suminc_stats* st) {
   c->stats.push_rounds = (double)h->rounds - (double)h->pull_rounds;
   const bool numeric_fail = h->aux[0] != 0;
   const double residual = h->residual;
-  pr_mass(c, &c->stats);
+  c->stats.mass_total = h->dpad[1];
+  c->stats.mass_defect = h->dpad[1] - h->dpad[2] - (1.0 - c->prm.damping);
   if (st) *st = c->stats;
   SUMINC_REQUIRE(!numeric_fail, SUMINC_E_NUMERIC, "NaN/Inf in PageRank residual");
   SUMINC_REQUIRE(!(residual >= T), SUMINC_E_NOT_CONVERGED, "round cap reached before sum|delta| < T");

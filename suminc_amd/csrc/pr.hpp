@@ -18,8 +18,6 @@ void pr_run(suminc_ctx* c, suminc_stats* st);
 void pr_step(suminc_ctx* c, double* residual);
 void pr_download(suminc_ctx* c, double* rank, double* delta);
 void pr_upload(suminc_ctx* c, const double* rank, const double* delta);
-// FP64 mass balance of the current PageRank state into st->mass_total / mass_defect
-void pr_mass(suminc_ctx* c, suminc_stats* st);
 unsigned push_grid();
 // clears the device counters on the stream (the start of a run)
 void zero_counters(suminc_ctx* c);

@@ -10,20 +10,20 @@
 
 namespace suminc {
 
-// Rows come from (off, col).  kSketch: a row of a clustered vertex (type[v] != 0,
-// i.e. an exit of the sketch) skips the edges that stay inside its cluster.
-template <class T, bool kSketch = false>
-__global__ void __launch_bounds__(kBlock) k_pr_push(const uint32_t* __restrict__ off, const uint32_t* __restrict__ col,
-                                                    T* __restrict__ delta, const uint32_t* __restrict__ wl_v,
-                                                    const T* __restrict__ wl_c, const uint4* __restrict__ heavy,
-                                                    const Counters* cnt, const uint8_t* __restrict__ type = nullptr,
-                                                    const uint32_t* __restrict__ cid = nullptr) {
+// The scatter of the calling grid; all its workgroups call it.  Rows come from (off,
+// col).  kSketch: a row of a clustered vertex (type[v] != 0, i.e. an exit of the sketch)
+// skips the edges that stay inside its cluster.
+template <class T, bool kSketch>
+__device__ __forceinline__ void pr_push_body(const uint32_t* __restrict__ off, const uint32_t* __restrict__ col,
+                                             T* __restrict__ delta, const uint32_t* __restrict__ wl_v,
+                                             const T* __restrict__ wl_c, const uint4* __restrict__ heavy,
+                                             const Counters* cnt, const uint8_t* __restrict__ type,
+                                             const uint32_t* __restrict__ cid) {
   __shared__ uint32_t s_scan[kBlock + 1];
   __shared__ uint32_t s_start[kBlock];
   __shared__ uint32_t s_warp[kBlock / 64 + 1];
   __shared__ T s_c[kBlock];
   __shared__ uint32_t s_k[kBlock];  // cluster of a clustered row, INF32 for a Single's row
-  if (cnt->done || cnt->mode != 0) return;
   const unsigned long long nl = cnt->wl_count[0];
   const unsigned long long nh = cnt->heavy_count;
   const uint32_t vt = frontier_tile<kBlock>(nl);
@@ -61,6 +61,17 @@ __global__ void __launch_bounds__(kBlock) k_pr_push(const uint32_t* __restrict__
       unsafeAtomicAdd(&delta[x], c);
     }
   }
+}
+
+// In push mode (mode 0) of a run that has not stopped.
+template <class T, bool kSketch = false>
+__global__ void __launch_bounds__(kBlock) k_pr_push(const uint32_t* __restrict__ off, const uint32_t* __restrict__ col,
+                                                    T* __restrict__ delta, const uint32_t* __restrict__ wl_v,
+                                                    const T* __restrict__ wl_c, const uint4* __restrict__ heavy,
+                                                    const Counters* cnt, const uint8_t* __restrict__ type = nullptr,
+                                                    const uint32_t* __restrict__ cid = nullptr) {
+  if (cnt->done || cnt->mode != 0) return;
+  pr_push_body<T, kSketch>(off, col, delta, wl_v, wl_c, heavy, cnt, type, cid);
 }
 
 }  // namespace suminc
