@@ -223,3 +223,38 @@ def plain_rounds_all(M, x, T):
     while np.abs(x).sum() >= T:
         x, k = M @ x, k + 1
     return k
+
+
+@pytest.mark.parametrize("n,m", [(2048, 32768), (2048, 32769), (2049, 32768), (2, 1), (1024, 1), (33, 1000)])
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+def test_runs_at_the_edge_of_one_workgroup(gpu, n, m, prec):
+    """Graphs of up to 2048 vertices and 32768 edges run in one workgroup, 512 rounds a
+    launch: at its limits and just beyond, to the fixed point and over 1100 rounds."""
+    rng = np.random.default_rng(n + m)
+    key = np.unique((n * rng.random(8 * m) ** 2).astype(np.int64) * n + rng.integers(0, n, 8 * m))
+    key = key[key // n != key % n]
+    key = np.sort(rng.permutation(key)[:m])
+    assert len(key) == min(m, n * (n - 1))
+    u, v = key // n, key % n
+    off = np.zeros(n + 1, np.uint64)
+    off[1:] = np.cumsum(np.bincount(u, minlength=n))
+    M = system(n, u, v)
+    x = np.full(n, (1 - DAMPING) / n)
+    want = limit(M, np.zeros(n), x)
+    T = 1e-11 if prec == "fp64" else 1e-7
+    p = gpu.PR_FP64 if prec == "fp64" else gpu.PR_FP32_KAHAN
+    with gpu.Context(pr_precision=p, termcheck_threshold=T, max_rounds=1000) as ctx:
+        ctx.upload_csr(off, v.astype(np.uint32))
+        ctx.pr_init()
+        st = ctx.pr_run()
+        r, d = ctx.pr_download()
+        assert st["residual"] < T and st["pull_rounds"] + st["push_rounds"] == st["rounds"]
+        assert np.abs(r - want).sum() <= T / (1 - DAMPING) + 0.15 * (1e-12 if prec == "fp64" else 1e-5)
+        assert abs(st["mass_defect"]) <= (1e-13 if prec == "fp64" else 1e-6)
+        if prec == "fp64" and m > 1000:
+            ctx.set_params(termcheck_threshold=0.0, max_rounds=1100)
+            ctx.pr_init()
+            st = ctx.pr_run(allow_not_converged=True)
+            r, d = ctx.pr_download()
+            assert st["rounds"] == 1100
+            assert np.abs(limit(M, r, d) - want).sum() <= 1e-13
