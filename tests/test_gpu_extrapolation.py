@@ -258,3 +258,60 @@ def test_runs_at_the_edge_of_one_workgroup(gpu, n, m, prec):
             r, d = ctx.pr_download()
             assert st["rounds"] == 1100
             assert np.abs(limit(M, r, d) - want).sum() <= 1e-13
+
+
+@pytest.mark.parametrize("div", [3, 1_000_000, 0], ids=["mixed", "pull", "push"])
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+def test_reseed_keeps_the_fixed_point(gpu, prec, div):
+    """After a batch rank and delta are a state of the new graph's fixed point: sources
+    that lose all edges, gain their first, swap edges at the same degree, only change
+    weights, or are named by deletes of nothing; also after a batch without pulls
+    between two with them (the pull's columns are not carried over it)."""
+    n, u, v, off = hubs()
+    rng = np.random.default_rng(21)
+    p = gpu.PR_FP64 if prec == "fp64" else gpu.PR_FP32_KAHAN
+    T = 1e-11 if prec == "fp64" else 1e-7
+    tol = 0.15 * (1e-12 if prec == "fp64" else 1e-5)
+    have = set(zip(u.tolist(), v.tolist()))
+
+    def ops(k):
+        deg = np.bincount([a for a, _ in have], minlength=n)
+        out = []
+        some = sorted(have)
+        lose = rng.choice(np.flatnonzero((deg > 0) & (deg < 4)), 40, replace=False)
+        for a in lose:  # every edge of some sources goes
+            out += [(1, a, b) for x, b in some if x == a]
+        none = np.flatnonzero(deg == 0)  # (from the second batch on: the first makes some)
+        for a in rng.choice(none, min(30, len(none)), replace=False) if len(none) else []:  # first edges
+            out += [(0, a, int(b)) for b in rng.integers(0, 300, 2) if b != a]
+        for i in rng.choice(len(some), 60, replace=False):  # an edge for another: the same degree
+            a, b = some[i]
+            c = int(rng.integers(0, n))
+            out += [(1, a, b)] + ([(0, a, c)] if c != a and (a, c) not in have else [])
+        for i in rng.choice(len(some), 20, replace=False):  # an add of an edge that is there
+            out.append((0, *some[i]))
+        for a, b in rng.integers(0, n, (20, 2)):  # a delete of one that is not
+            if (a, b) not in have and a != b:
+                out.append((1, int(a), int(b)))
+        rec = np.zeros(len(out), gpu.UPDATE_DTYPE)
+        rec["type"], rec["u"], rec["v"] = np.array(out).T
+        adds = {(a, b) for t, a, b in out if t == 0}
+        return rec, (have - {(a, b) for t, a, b in out if t == 1}) | adds
+
+    with gpu.Context(pr_precision=p, termcheck_threshold=T, max_rounds=1000, pull_threshold_div=div,
+                     pull_compact_kib=1) as ctx:
+        ctx.upload_csr(off, v.astype(np.uint32))
+        ctx.pr_init()
+        ctx.pr_run()
+        for k in range(4):
+            rec, have = ops(k)
+            ctx.set_params(pull_threshold_div=0 if k == 1 else div)
+            ctx.apply_batch(rec)
+            a, b = np.array(sorted(have)).T
+            M = system(n, a, b)
+            want = limit(M, np.zeros(n), np.full(n, (1 - DAMPING) / n))
+            r, d = ctx.pr_download()
+            assert np.abs(limit(M, r, d) - want).sum() <= tol
+            ctx.pr_run()
+            r, _ = ctx.pr_download()
+            assert np.abs(r - want).sum() <= T / (1 - DAMPING) + tol
