@@ -85,7 +85,7 @@ struct DevBuf {
 // the block's run); the value stream (one element per edge); optionally the row
 // order's index of every edge (eid) and a coefficient per edge in layout order.
 struct BinLayout {
-  DevBuf packed, packed2, eid, eid2, F2, F, hist, pieces, parts, vals, bounds, coef;
+  DevBuf packed, packed2, eid, eid2, F2, F, hist, pieces, parts, vals, bounds, coef, seg0;
   uint32_t n_parts = 0, P = 0, B = 0, wl = 0, bsize = 0, direct = 0;
   uint64_t first = 0, m = 0;  // the value stream's edges: [first, m)
 };

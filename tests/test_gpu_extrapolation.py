@@ -81,6 +81,15 @@ def limit(M, r, x):
     return r + sla.spsolve(sp.eye(M.shape[0], format="csc") - M.tocsc(), x)
 
 
+def series_limit(M, x):
+    """The same for larger graphs, whose factors fill in: the series to 2^-60."""
+    r = x.copy()
+    while np.abs(x).sum() > 1e-18:
+        x = M @ x
+        r += x
+    return r
+
+
 GRAPHS = ["one", "ring", "pairs", "path", "grid", "communities", "uniform", "skewed"]
 
 
@@ -315,3 +324,38 @@ def test_reseed_keeps_the_fixed_point(gpu, prec, div):
             ctx.pr_run()
             r, _ = ctx.pr_download()
             assert np.abs(r - want).sum() <= T / (1 - DAMPING) + tol
+
+
+@pytest.mark.parametrize("n,m", [(3000, 16383), (3000, 16384), (3000, 16385), (9000, 49157), (200_000, 100_000),
+                                 (200_000, 400_000)])
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+def test_binned_layout_at_the_edges_of_its_sort_tiles(gpu, n, m, prec):
+    """The binned pull (1 KiB windows) with layouts around whole sort tiles (16384 edges,
+    8192 with coefficients), a few segments a tile and more than a tile's counters."""
+    rng = np.random.default_rng(m)
+    key = np.unique((n * rng.random(2 * m) ** 3).astype(np.int64) * n + (n * rng.random(2 * m) ** 2).astype(np.int64))
+    key = key[key // n != key % n]
+    key = np.sort(rng.permutation(key)[:m])
+    assert len(key) == m
+    u, v = key // n, key % n
+    off = np.zeros(n + 1, np.uint64)
+    off[1:] = np.cumsum(np.bincount(u, minlength=n))
+    w = (1.0 - rng.random(m)).astype(np.float32)
+    M = system(n, u, v)
+    s = np.bincount(u, weights=w.astype(float), minlength=n)
+    W = sp.csr_matrix((DAMPING * w.astype(float) / s[u], (v, u)), shape=(n, n))
+    T = 1e-11 if prec == "fp64" else 1e-7
+    tol = 0.15 * (1e-12 if prec == "fp64" else 1e-5)
+    p = gpu.PR_FP64 if prec == "fp64" else gpu.PR_FP32_KAHAN
+    x = np.full(n, 1.0 / n, np.float32)
+    with gpu.Context(pr_precision=p, termcheck_threshold=T, max_rounds=1000, pull_bin_kib=1) as ctx:
+        ctx.upload_csr(off, v.astype(np.uint32), w)
+        ctx.pr_init()
+        ctx.pr_run()
+        r, _ = ctx.pr_download()
+        ctx.wpr_set_weights(w)
+        rw, _ = ctx.wpr_forward(x)
+    want = series_limit(M, np.full(n, (1 - DAMPING) / n))
+    assert np.abs(r - want).sum() <= T / (1 - DAMPING) + tol
+    want = series_limit(W, (1 - DAMPING) * x.astype(float))
+    assert np.abs(rw - want).sum() <= T / (1 - DAMPING) + 0.15 * 1e-5  # comes back as FP32
