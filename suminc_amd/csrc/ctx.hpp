@@ -182,6 +182,7 @@ struct Sketch {
   DevBuf sc_R, sc_D;         // PageRank rows (reach mass / residual) per entry
   DevBuf ss_dist;            // SSSP rows (in-cluster distance to every exit) per entry
   DevBuf bound, spnode;      // PageRank sketch accumulators
+  DevBuf pr_work;            // u64: internal edges read by the row build, then by the precompute
   DevBuf ex_taken;           // inflow each exit turned into rank in the last round
   DevBuf xi_list, xi_count;  // internal edges leaving exits: (contribution slot of the exit, destination)
   DevBuf exits, exit_count;  // the exits of the current layout (sketch rounds' exit pass)

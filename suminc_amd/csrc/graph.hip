@@ -109,8 +109,9 @@ void build_csc(suminc_ctx* c) {
   const uint64_t m = c->m;
   const uint32_t n = c->n;
   c->in_off.ensure(((size_t)n + 1) * 4);
-  c->in_col.ensure(m * 4 + 4);
-  if (c->wkind) c->in_w.ensure(m * 4 + 4);
+  // with headroom: a batch swaps these with its workspace, and grown graphs fit them
+  c->in_col.ensure_slack(m * 4 + 4);
+  if (c->wkind) c->in_w.ensure_slack(m * 4 + 4);
   if (m == 0) {
     SUMINC_HIP(hipMemsetAsync(c->in_off.p, 0, ((size_t)n + 1) * 4, c->stream));
     return;
@@ -202,8 +203,8 @@ void generate_rmat(suminc_ctx* c, int scale, int edge_factor, double a, double b
   c->m = m;
   c->wkind = wkind;
   c->out_off.ensure(((size_t)n + 1) * 4);
-  c->out_col.ensure(m * 4 + 4);
-  if (wkind) c->out_w.ensure(m * 4 + 4);
+  c->out_col.ensure_slack(m * 4 + 4);
+  if (wkind) c->out_w.ensure_slack(m * 4 + 4);
   k_keys_to_cols<<<grid_for(m), kBlock, 0, c->stream>>>(keys_a.as<uint64_t>(), m, scale, c->out_col.as<uint32_t>(),
                                                         wkind, wmin, wmax, k0, k1, c->out_w.p);
   k_row_pointers<<<grid_for(m + 1), kBlock, 0, c->stream>>>(keys_a.as<uint64_t>(), m, scale, n,
@@ -235,8 +236,8 @@ void upload_csr(suminc_ctx* c, uint32_t n, uint64_t m, const uint64_t* off, cons
   c->m = m;
   c->wkind = wkind;
   c->out_off.ensure(((size_t)n + 1) * 4);
-  c->out_col.ensure(m * 4 + 4);
-  if (wkind) c->out_w.ensure(m * 4 + 4);
+  c->out_col.ensure_slack(m * 4 + 4);
+  if (wkind) c->out_w.ensure_slack(m * 4 + 4);
   std::vector<uint32_t> off32(n + 1);
   for (uint32_t i = 0; i <= n; ++i) off32[i] = (uint32_t)off[i];
   SUMINC_HIP(hipMemcpyAsync(c->out_off.p, off32.data(), ((size_t)n + 1) * 4, hipMemcpyHostToDevice, c->stream));

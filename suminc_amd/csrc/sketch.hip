@@ -1328,7 +1328,7 @@ static void compute_pr_rows(suminc_ctx* c) {
     s.sc_R.ensure_slack(s.sc_len * es + es);
     s.sc_D.ensure_slack(s.sc_len * es + es);
   }
-  DevBuf work;
+  DevBuf& work = s.pr_work;
   work.ensure(8);
   SUMINC_HIP(hipMemsetAsync(work.p, 0, 8, c->stream));
   const double thr_pv = c->prm.termcheck_threshold / (double)c->n;  // T / N_old * |C| per cluster
@@ -1963,7 +1963,7 @@ static void sum_pr_run_t(suminc_ctx* c, suminc_stats* st) {
   a.partial = c->partial.as<double>();
   a.cid = s.cid.as<uint32_t>();
   a.cl_nexit = s.cl_nexit.as<uint32_t>();
-  DevBuf work;
+  DevBuf& work = s.pr_work;
   work.ensure(8);
   SUMINC_HIP(hipMemsetAsync(work.p, 0, 8, c->stream));
   suminc_stats out{};
