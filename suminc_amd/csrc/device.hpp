@@ -48,6 +48,13 @@ __device__ __forceinline__ unsigned long long wave_append(bool pred, unsigned lo
   return base + __popcll(below);
 }
 
+// Orders this wave's LDS traffic before what follows (wave-local exchange).
+__device__ __forceinline__ void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // Block-wide exclusive scan of one uint32 per thread (blockDim.x == BLOCK).
 template <int BLOCK>
 __device__ __forceinline__ uint32_t block_exclusive_scan(uint32_t v, uint32_t* lds_warp, uint32_t* total) {

@@ -1772,7 +1772,8 @@ __global__ void k_lists_clear(Counters* cnt) {
   cnt->mode = 0;
 }
 
-// Precompute of one dirty cluster per workgroup: the members' pending delta is
+// Precompute of one dirty cluster of more than kWaveCluster members per workgroup (those
+// in `large`; the others: k_sk_precompute_small): the members' pending delta is
 // iterated inside the cluster (run_to_convergence_for_precpt), the mass that
 // arrived becomes rank, the residual stays in delta, and every exit sends d/outdeg
 // of its arrived mass over its external edges (first_step, :389-434): the exit's
@@ -1780,7 +1781,8 @@ __global__ void k_lists_clear(Counters* cnt) {
 // into rank and sends it with that round's scatter.  Dissolved clusters are
 // Singles and are not iterated.
 template <class T>
-__global__ void __launch_bounds__(kBlock) k_sk_precompute(SkArgs a, const uint32_t* __restrict__ cl_off,
+__global__ void __launch_bounds__(kBlock) k_sk_precompute(const uint32_t* __restrict__ large,
+                                                          const uint32_t* __restrict__ cl_off,
                                                           const uint32_t* __restrict__ cl_mem,
                                                           const uint32_t* __restrict__ cl_nexit, Internal ie,
                                                           uint8_t* dirty, const uint8_t* __restrict__ dead,
@@ -1790,7 +1792,7 @@ __global__ void __launch_bounds__(kBlock) k_sk_precompute(SkArgs a, const uint32
                                                           unsigned long long* work) {
   __shared__ T s_r[kMaxCluster], s_d[kMaxCluster], s_n[kMaxCluster];
   __shared__ T s_red[kBlock / 64];
-  const uint32_t k = blockIdx.x;
+  const uint32_t k = large[blockIdx.x];
   if (!dirty[k]) return;
   if (dead[k]) {
     if (threadIdx.x == 0) dirty[k] = 0;
@@ -1817,6 +1819,87 @@ __global__ void __launch_bounds__(kBlock) k_sk_precompute(SkArgs a, const uint32
     dirty[k] = 0;
     atomicAdd(work, (unsigned long long)rounds * (pe - pb));
   }
+}
+
+// The same for the dirty clusters of at most kWaveCluster members, one per wave: member
+// j's delta and rank in lane j's registers, the exchange in LDS, up to 128 internal edges
+// in registers across the rounds, no workgroup barrier.  A round of such a cluster moves
+// a few hundred bytes, so a workgroup each spent its time on launches and barriers: a 1%
+// batch on 2^26 vertices 5.33 -> 0.67 ms, on 2^24 1.50 -> 0.25.
+constexpr unsigned kPrecomputeGrid = 2048;
+template <class T>
+__global__ void __launch_bounds__(kBlock) k_sk_precompute_small(
+    uint32_t K, const uint32_t* __restrict__ cl_off, const uint32_t* __restrict__ cl_mem,
+    const uint32_t* __restrict__ cl_nexit, Internal ie, uint8_t* dirty, const uint8_t* __restrict__ dead,
+    T* __restrict__ delta, T* __restrict__ rank, float* __restrict__ comp, T* __restrict__ bound, T d,
+    double thr_per_vertex, int maxit, unsigned long long* work) {
+  __shared__ T s_d[kBlock / 64][64], s_n[kBlock / 64][64];
+  __shared__ unsigned long long s_work;
+  if (threadIdx.x == 0) s_work = 0;
+  __syncthreads();
+  const uint32_t wv = threadIdx.x >> 6, lane = lane_id();
+  unsigned long long read = 0;
+  for (uint32_t k = blockIdx.x * (kBlock / 64) + wv; k < K; k += gridDim.x * (kBlock / 64)) {
+    if (!dirty[k]) continue;
+    const uint32_t slot0 = cl_off[k], size = cl_off[k + 1] - slot0;
+    if (size > kWaveCluster) continue;
+    if (dead[k]) {
+      if (lane == 0) dirty[k] = 0;
+      continue;
+    }
+    const uint32_t pb = ie.off[k], pe = ie.off[k + 1], v = lane < size ? cl_mem[slot0 + lane] : 0u;
+    T dv = lane < size ? delta[v] : T(0), r = T(0);
+    uint32_t es[2] = {0, 0}, et[2] = {0, 0}, eg[2] = {1, 1};
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const uint32_t p = pb + lane + 64 * j;
+      if (p < pe) {
+        es[j] = ie.src[p];
+        et[j] = ie.dst[p];
+        eg[j] = ie.deg[p];
+      }
+    }
+    const double thr = thr_per_vertex * size;
+    uint32_t rounds = 0;
+    for (int it = 0; it < maxit; ++it) {
+      s_d[wv][lane] = dv;
+      s_n[wv][lane] = T(0);
+      wave_lds_sync();
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        if (pb + lane + 64 * j >= pe) continue;
+        const T x = s_d[wv][es[j]];
+        if (x != T(0)) atomicAdd(&s_n[wv][et[j]], x * d / (T)eg[j]);
+      }
+      for (uint32_t p = pb + 128 + lane; p < pe; p += 64) {
+        const T x = s_d[wv][ie.src[p]];
+        if (x != T(0)) atomicAdd(&s_n[wv][ie.dst[p]], x * d / (T)ie.deg[p]);
+      }
+      T tot = fabs_t(dv);
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1) tot += __shfl_xor(tot, o);
+      wave_lds_sync();
+      r += dv;
+      dv = s_n[wv][lane];
+      wave_lds_sync();
+      ++rounds;
+      if ((double)tot <= thr) break;
+    }
+    if (lane < size) {
+      delta[v] = dv;
+      if (r != T(0)) {
+        if (lane < cl_nexit[k]) bound[v] += r;  // sent by the next exit pass
+        else kahan_add(rank, comp, v, r);
+      }
+    }
+    if (lane == 0) {
+      dirty[k] = 0;
+      read += (unsigned long long)rounds * (pe - pb);
+    }
+  }
+  if (read) atomicAdd(&s_work, read);
+  __syncthreads();
+  if (threadIdx.x == 0 && s_work) atomicAdd(work, s_work);
 }
 
 // Correction (sum_sync_iter_worker.h:1414-1469): the delta accumulated at every
@@ -1972,12 +2055,15 @@ static void sum_pr_run_t(suminc_ctx* c, suminc_stats* st) {
   zero_counters(c);
   k_lists_clear<<<1, 64, 0, c->stream>>>(cnt);
   if (s.K)
-    k_sk_precompute<T><<<s.K, kBlock, 0, c->stream>>>(a, s.cl_off.as<uint32_t>(), s.cl_mem.as<uint32_t>(),
-                                                      s.cl_nexit.as<uint32_t>(), internal_of(s),
-                                                      s.dirty.as<uint8_t>(), s.dead.as<uint8_t>(),
-                                                      c->pr_delta.as<T>(), c->pr_rank.as<T>(),
-                                                      c->pr_comp.as<float>(), s.bound.as<T>(), d, eps, maxit,
-                                                      work.as<unsigned long long>());
+    k_sk_precompute_small<T><<<std::min<uint32_t>((s.K + kWaves - 1) / kWaves, kPrecomputeGrid), kBlock, 0, c->stream>>>(
+        s.K, s.cl_off.as<uint32_t>(), s.cl_mem.as<uint32_t>(), s.cl_nexit.as<uint32_t>(), internal_of(s),
+        s.dirty.as<uint8_t>(), s.dead.as<uint8_t>(), c->pr_delta.as<T>(), c->pr_rank.as<T>(), c->pr_comp.as<float>(),
+        s.bound.as<T>(), d, eps, maxit, work.as<unsigned long long>());
+  if (s.n_large)
+    k_sk_precompute<T><<<s.n_large, kBlock, 0, c->stream>>>(
+        s.large.as<uint32_t>(), s.cl_off.as<uint32_t>(), s.cl_mem.as<uint32_t>(), s.cl_nexit.as<uint32_t>(),
+        internal_of(s), s.dirty.as<uint8_t>(), s.dead.as<uint8_t>(), c->pr_delta.as<T>(), c->pr_rank.as<T>(),
+        c->pr_comp.as<float>(), s.bound.as<T>(), d, eps, maxit, work.as<unsigned long long>());
   k_lists_clear<<<1, 64, 0, c->stream>>>(cnt);
   SUMINC_HIP(hipGetLastError());
   // the exits of this layout, for the rounds' exit pass

@@ -139,13 +139,6 @@ __global__ void __launch_bounds__(kBlock) k_cluster_lists(uint32_t K, const uint
   else if (large) list[K - 1 - (bl + __popcll(ml & below))] = k;
 }
 
-// Orders this wave's LDS traffic before what follows (wave-local exchange).
-__device__ __forceinline__ void wave_lds_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // cluster_bf for a cluster of at most 64 members run by one wave (s_id, s_dp are
 // this wave's LDS slots): up to 128 internal edges stay in registers across the
 // rounds; a round ends with a wave vote instead of workgroup barriers.
