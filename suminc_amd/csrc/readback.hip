@@ -6,9 +6,8 @@
 // result crosses in chunks: a kernel converts the state and stores a chunk straight to a
 // pinned slot, an event says that it is there, and several threads copy the slots to the
 // caller's array while the next chunks cross.  MI355X, FP32 state of 2^26 vertices to two
-// FP64 arrays (1 GiB): 104 -> 23
-// ms; 2^22 vertices, distances and parents (32 MiB): 2.5 -> 1.3 ms; 1000 vertices, 84 -> 50 us
-// (no allocation).
+// FP64 arrays (1 GiB): 104 -> 23 ms; 2^22 vertices, distances and parents (32 MiB):
+// 2.5 -> 0.95 ms; 1000 vertices: 84 -> 50 us (no allocation).
 #include "readback.hpp"
 
 #include <atomic>

@@ -330,8 +330,8 @@ def test_reseed_keeps_the_fixed_point(gpu, prec, div):
                                  (200_000, 400_000)])
 @pytest.mark.parametrize("prec", ["fp64", "fp32"])
 def test_binned_layout_at_the_edges_of_its_sort_tiles(gpu, n, m, prec):
-    """The binned pull (1 KiB windows) with layouts around whole sort tiles (16384 edges,
-    8192 with coefficients), a few segments a tile and more than a tile's counters."""
+    """The binned pull (1 KiB windows) with layouts around whole steps of the ordering
+    (8192 edges), a few segments a workgroup and more than its 4096 counters."""
     rng = np.random.default_rng(m)
     key = np.unique((n * rng.random(2 * m) ** 3).astype(np.int64) * n + (n * rng.random(2 * m) ** 2).astype(np.int64))
     key = key[key // n != key % n]
