@@ -60,9 +60,9 @@ __device__ __forceinline__ void sssp_relax(const SsspArgs& a, int nxt, uint32_t 
     unsigned long long cand = (nd << 32) | u;
     // words only decrease while the rounds run: a candidate no smaller than a
     // plain (possibly stale) read cannot win, so it skips the atomic.  SSWP takes
-    // strictly better words only (no parent change on a tie: no parent cycles)
+    // strictly better values only (trav_commit)
     if (a.app == SUMINC_APP_SSWP ? nd < (a.dp[v] >> 32) : cand < a.dp[v]) {
-      unsigned long long old = atomicMin(&a.dp[v], cand);
+      unsigned long long old = trav_commit(a.app, &a.dp[v], cand);
       add = (old >> 32) > nd;
     }
   }
@@ -209,7 +209,7 @@ __global__ void __launch_bounds__(kBlock) k_sssp_pull(SsspArgs a, SsspPull p) {
       if (nd >= INF32) continue;
       const unsigned long long cand = nd << 32 | u, was = a.dp[lo];
       if (!sssp_better(a.app, cand, was, (uint32_t)(was >> 32))) continue;
-      if ((atomicMin(&a.dp[lo], cand) >> 32) > nd) sssp_mark(a.bits[nxt], lo);
+      if ((trav_commit(a.app, &a.dp[lo], cand) >> 32) > nd) sssp_mark(a.bits[nxt], lo);
     }
   } else {
 #pragma unroll
@@ -297,7 +297,7 @@ __global__ void __launch_bounds__(kBlock) k_sssp_pull(SsspArgs a, SsspPull p) {
       if (p.ioff[v] >= e0 && p.ioff[v + 1] <= e0 + ne) {
         a.dp[v] = best;
         if ((uint32_t)(best >> 32) < s_old[i]) sssp_mark(a.bits[nxt], v);
-      } else if ((atomicMin(&a.dp[v], best) >> 32) > (best >> 32)) {
+      } else if ((trav_commit(a.app, &a.dp[v], best) >> 32) > (best >> 32)) {
         sssp_mark(a.bits[nxt], v);
       }
     }

@@ -108,3 +108,40 @@ def test_pull_rounds_reach_the_fixed_point(gpu, name, app):
     for _ in range(int(n).bit_length()):
         up = up[up]
     assert (up[reached] == 0).all()
+
+
+def test_widths_with_many_ties_keep_a_tree_of_parents(gpu):
+    """SSWP on three widths: rows of 10,000 in-edges, each over many tiles and nearly all
+    of them ties, from scratch and after a batch that deletes every hub's parent edge."""
+    rng = np.random.default_rng(8)
+    n, hubs = 50_000, 60
+    u = np.concatenate([rng.integers(0, n, 600_000), rng.integers(0, hubs, 200_000), np.zeros(60, int)])
+    v = np.concatenate([rng.integers(0, hubs, 600_000), rng.integers(0, n, 200_000), rng.integers(0, n, 60)])
+    off, col, w, u, v = csr(n, u, v, rng, 3)
+
+    def check(val, par, u, v, w):
+        d, c = relax(n, u, v, w, "sswp")
+        assert np.array_equal(INF - val.astype(np.int64), d)
+        reached = (d < INF) & (np.arange(n) > 0)
+        ok = np.zeros(n, bool)
+        ok[v[(c == d[v]) & (par[v] == u)]] = True
+        assert ok[reached].all()
+        up = np.where(reached, par, 0).astype(np.int64)
+        for _ in range(int(n).bit_length()):
+            up = up[up]
+        assert (up[reached] == 0).all()
+
+    with gpu.Context() as ctx:
+        ctx.upload_csr(off, col, w)
+        ctx.traversal_init(gpu.APP_SSWP, 0)
+        assert ctx.sssp_run()["pull_rounds"] >= 1
+        val, par = ctx.sssp_download()
+        check(val, par, u, v, w)
+        gone = np.isin(u * n + v, [int(par[h]) * n + h for h in range(1, hubs)])
+        rec = np.zeros(gone.sum(), gpu.UPDATE_DTYPE)
+        rec["type"], rec["u"], rec["v"] = 1, u[gone], v[gone]
+        assert len(rec) > hubs // 2
+        ctx.apply_batch(rec)
+        ctx.sssp_run()
+        val, par = ctx.sssp_download()
+        check(val, par, u[~gone], v[~gone], w[~gone])
