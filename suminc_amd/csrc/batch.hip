@@ -452,7 +452,13 @@ __global__ void k_gather_groups(const uint32_t* sidx, const unsigned* bc, const 
 //   (k_reseed_fix, per group),
 // so one pass over the new graph does for both: a 1% batch on 2^26 vertices took two
 // pulls (4.5 ms each) and two lists (2.0 ms), now one of each and 0.8 ms of corrections.
-// A source whose degree stays sends nothing along its kept edges.
+// A source whose degree stays sends nothing along its kept edges.  In FP32 the two terms
+// of an inserted edge leave d r_u / deg_old * 2^-24 behind, the same along all of them, so
+// a source whose degree more than doubles sends the two amendments as they stand:
+//   d r_u / deg_new along every new edge (k_reseed_list),
+//   - d r_u / deg_old along every old one (k_reseed_fix): it has more groups than old
+//   edges, and its i-th group takes the i-th.
+__device__ __forceinline__ bool reseed_grown(uint32_t was, uint32_t deg) { return deg > was && deg - was > was; }
 __device__ __forceinline__ double reseed_rank(const double* rank, const float*, uint32_t u) { return rank[u]; }
 __device__ __forceinline__ double reseed_rank(const float* rank, const float* comp, uint32_t u) {
   return (double)rank[u] - (double)comp[u];
@@ -477,7 +483,7 @@ __global__ void __launch_bounds__(kBlock) k_reseed_list(const uint32_t* t_list, 
     const uint32_t deg = off[u + 1] - off[u], was = off_old[u + 1] - off_old[u];
     if (deg > 0 && deg != was) {
       const double dr = d * reseed_rank(rank, comp, u);
-      c = (T)(dr / deg - (was ? dr / was : 0.0));
+      c = (T)(dr / deg - (was && !reseed_grown(was, deg) ? dr / was : 0.0));
     }
     if (c != T(0)) {
       contrib[pos ? pos[u] : u] = c;  // deg > 0: u has a position
@@ -511,16 +517,28 @@ template <class T>
 __global__ void __launch_bounds__(kBlock) k_reseed_fix(const uint32_t* __restrict__ row, const uint32_t* __restrict__ col,
                                                        const uint8_t* __restrict__ act, const uint8_t* __restrict__ ex,
                                                        const unsigned* bc, uint32_t N,
-                                                       const uint32_t* __restrict__ off_old, const T* rank,
+                                                       const uint32_t* __restrict__ tix,
+                                                       const uint32_t* __restrict__ t_gbeg,
+                                                       const uint32_t* __restrict__ off_old,
+                                                       const uint32_t* __restrict__ col_old,
+                                                       const uint32_t* __restrict__ off, const T* rank,
                                                        const float* comp, double d, T* __restrict__ delta) {
   const uint32_t g = blockIdx.x * kBlock + threadIdx.x;
   if (g >= N || g >= bc[0]) return;
-  const bool add = act[g] == 0, existed = ex[g];
-  if (add == existed) return;  // a weight replaced, or a delete of nothing
-  const uint32_t u = row[g], was = off_old[u + 1] - off_old[u];
+  const uint32_t u = row[g], b = off_old[u], was = off_old[u + 1] - b;
   if (!was) return;
+  bool add = act[g] == 0;
+  uint32_t v = col[g];
+  if (reseed_grown(was, off[u + 1] - off[u])) {
+    const uint32_t i = g - t_gbeg[tix[u]];
+    if (i >= was) return;
+    add = false;
+    v = col_old[b + i];
+  } else if (add == (ex[g] != 0)) {
+    return;  // a weight replaced, or a delete of nothing
+  }
   const T c = (T)(d * reseed_rank(rank, comp, u) / was);
-  if (c != T(0)) unsafeAtomicAdd(&delta[col[g]], add ? c : -c);
+  if (c != T(0)) unsafeAtomicAdd(&delta[v], add ? c : -c);
 }
 
 // Scatter of the reseed: pull over the CSC when its edges exceed m / div (the
@@ -941,9 +959,9 @@ static void merge_direction(suminc_ctx* c, DevBuf& off, DevBuf& col, DevBuf& w, 
   if (colc) colc->swap(*ncolc);
 }
 
-// The reseed of the touched sources (after the CSR merge: b.noff_out holds the old row
-// pointers): push for a few edges, or, when they exceed m / div, one pull over the CSC
-// (whose work lists must be current: `lists` false leaves the pull out).
+// The reseed of the touched sources (after the CSR merge: b.noff_out and b.ncol_out hold
+// the old rows): push for a few edges, or, when they exceed m / div, one pull over the
+// CSC (whose work lists must be current: `lists` false leaves the pull out).
 template <class T>
 static void pr_reseed(suminc_ctx* c, uint32_t N, bool lists) {
   Counters* cnt = dev_counters(c);
@@ -965,7 +983,9 @@ static void pr_reseed(suminc_ctx* c, uint32_t N, bool lists) {
   if (div > 0) pull_scatter<T>(c, 1);
   k_reseed_fix<T><<<grid_for(N), kBlock, 0, c->stream>>>(b.g_row.as<uint32_t>(), b.g_col.as<uint32_t>(),
                                                          b.g_act.as<uint8_t>(), b.g_ex.as<uint8_t>(),
-                                                         b.bc.as<unsigned>(), N, off_old, c->pr_rank.as<T>(),
+                                                         b.bc.as<unsigned>(), N, b.tix.as<uint32_t>(),
+                                                         b.t_gbeg.as<uint32_t>(), off_old, b.ncol_out.as<uint32_t>(),
+                                                         c->out_off.as<uint32_t>(), c->pr_rank.as<T>(),
                                                          c->pr_comp.as<float>(), c->prm.damping, c->pr_delta.as<T>());
   k_reset_lists<<<1, 64, 0, c->stream>>>(cnt);
   SUMINC_HIP(hipGetLastError());

@@ -326,6 +326,59 @@ def test_reseed_keeps_the_fixed_point(gpu, prec, div):
             assert np.abs(r - want).sum() <= T / (1 - DAMPING) + tol
 
 
+@pytest.mark.parametrize("div", [1_000_000, 0], ids=["pull", "push"])
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+def test_reseed_of_sources_that_gain_many_edges(gpu, prec, div):
+    """Sources of high rank whose degree grows by factors from just below to far above two,
+    some losing old edges besides.  The batch itself is held against the exact amendment of
+    the state it found: every amended edge takes at most three roundings of a term of its
+    source's mass (the contribution, the two additions), so the deltas' error stays under
+    eps * 3 * (the mass that the sources sent before and send now + sum |delta|)."""
+    rng = np.random.default_rng(17)
+    n, k = 6007, 12
+    grow = [(1, 5000), (1, 3), (1, 2), (3, 7), (3, 6), (100, 200), (100, 201), (100, 5000), (700, 1401), (2, 300),
+            (300, 290), (5, 0)]
+    u = [np.arange(100, n)]  # everybody points at one of the sources
+    v = [rng.integers(0, k, n - 100)]
+    for s, (a, _) in enumerate(grow):
+        u.append(np.full(a, s))
+        v.append(rng.choice(np.arange(100, n), a, replace=False))
+    key = np.unique(np.concatenate(u) * n + np.concatenate(v))
+    u, v = key // n, key % n
+    off = np.zeros(n + 1, np.uint64)
+    off[1:] = np.cumsum(np.bincount(u, minlength=n))
+    ops, have = [], set(key.tolist())
+    for s, (a, b) in enumerate(grow):
+        row = v[u == s]
+        assert len(row) == a
+        lost = row[: min(a, s % 3 if b > a else a - b)]
+        ops += [(1, s, int(t)) for t in lost]
+        new = np.setdiff1d(np.arange(100, n), row)
+        ops += [(0, s, int(t)) for t in rng.choice(new, max(0, b - a + len(lost)), replace=False)]
+        if b > a and len(row) > len(lost):
+            ops.append((0, s, int(row[-1])))  # an add of an edge that is there
+    rec = np.zeros(len(ops), gpu.UPDATE_DTYPE)
+    rec["type"], rec["u"], rec["v"] = np.array(ops).T
+    rec = rng.permutation(rec)
+    have = (have - {a * n + b for t, a, b in ops if t == 1}) | {a * n + b for t, a, b in ops if t == 0}
+    a, b = np.divmod(np.array(sorted(have)), n)
+    assert [int((a == s).sum()) for s in range(k)] == [g for _, g in grow]
+    M0, M1 = system(n, u, v), system(n, a, b)
+    p = gpu.PR_FP64 if prec == "fp64" else gpu.PR_FP32_KAHAN
+    eps = 2.0 ** (-53 if prec == "fp64" else -24)
+    with gpu.Context(pr_precision=p, termcheck_threshold=1e-6, max_rounds=1000, pull_threshold_div=div) as ctx:
+        ctx.upload_csr(off, v.astype(np.uint32))
+        ctx.pr_init()
+        ctx.pr_run()
+        r, d = ctx.pr_download()
+        ctx.apply_batch(rec)
+        r1, d1 = ctx.pr_download()
+    assert np.array_equal(r, r1) and r[0] > 0.02
+    sent = DAMPING * r[:k].sum()
+    want = d + (M1 - M0) @ r
+    assert np.abs(d1 - want).sum() <= eps * 3 * (2 * sent + np.abs(d).sum() + np.abs(want).sum())
+
+
 @pytest.mark.parametrize("n,m", [(3000, 16383), (3000, 16384), (3000, 16385), (9000, 49157), (200_000, 100_000),
                                  (200_000, 400_000)])
 @pytest.mark.parametrize("prec", ["fp64", "fp32"])
