@@ -45,6 +45,7 @@
 #include "pr.hpp"
 #include "readback.hpp"
 #include "push.hpp"
+#include "sort_tiles.hpp"
 
 namespace suminc {
 
@@ -1556,8 +1557,8 @@ __global__ void __launch_bounds__(kBlock) k_bin_hist(const uint4* __restrict__ p
   const uint4 t = pieces[blockIdx.x];
   for (uint32_t w = threadIdx.x; w < P + kHotSubs - 1; w += kBlock) s_h[w] = 0;
   __syncthreads();
-  for (uint32_t e0 = t.z; e0 < t.w; e0 += kBlock) {  // the same trip count for every lane (ballots)
-    const uint32_t e = e0 + threadIdx.x;
+  for (uint64_t e0 = t.z; e0 < t.w; e0 += kBlock) {  // the same trip count for every lane (ballots)
+    const uint64_t e = e0 + threadIdx.x;
     const uint32_t w = e < t.w ? bin_key(icol[e], wl) : INF32;
     const unsigned long long hot = __ballot(w == 0);
     if (lane_id() == 0 && hot) atomicAdd(&s_h[0], (uint32_t)__popcll(hot));
@@ -1904,9 +1905,6 @@ __global__ void __launch_bounds__(kBinBlock) k_pr_bin_sum(const uint4* __restric
 // one write of the edges replace a segmented radix sort of 19 bits: 1.06G edges
 // 16.0 -> 3.7 ms (and the placing 0.9 ms more), a round over them 4.43 -> 4.56 ms, and a batch's layout
 // serves about nine rounds.
-constexpr int kSortBlock = 1024, kSortPer = 16;
-constexpr uint32_t kSortTile = kSortPer * kSortBlock - 4;  // a chunk may begin up to 3 edges into its first 16 bytes
-constexpr uint32_t kSortStep = 8192, kSortBins = 4096;
 
 // seg0[t]: the first segment that begins at edge t * kSortStep or after it (F2: nseg + 1
 // segment offsets)
@@ -1931,16 +1929,16 @@ __global__ void __launch_bounds__(kSortBlock) k_bin_sort(const uint32_t* __restr
   const uint32_t t = threadIdx.x, g0 = seg0[blockIdx.x], g1 = seg0[blockIdx.x + 1];
   if (g0 == g1 || g1 - g0 > kSortBins) return;  // more segments than counters: nothing to order in them
   const uint32_t nb = kSortBins / (g1 - g0), stop = F2[g1];
-  for (uint32_t lo = F2[g0]; lo < stop; lo += kSortTile) {
-    const uint32_t hi = stop - lo < kSortTile ? stop : lo + kSortTile;
-    // this thread's consecutive edges [i0, i0 + kSortPer), those of [lo, hi); the reads
-    // stay below hi + 3 (the array ends 16 bytes later)
-    const uint32_t i0 = (lo & ~3u) + t * kSortPer;
+  for (uint32_t lo = F2[g0], hi; lo < stop; lo = hi) {
+    hi = sort_chunk_end(lo, stop);
+    // this thread's consecutive edges base + [o0, o0 + kSortPer), those of [lo, hi); the
+    // reads stay below hi + 3 (the array ends 16 bytes later)
+    const uint32_t base = lo & ~3u, len = hi - base, o0 = t * kSortPer;
     uint32_t x[kSortPer], at[kSortPer];  // at: counter << 16 | the edge's turn there
 #pragma unroll
     for (int j = 0; j < kSortPer / 4; ++j) {
       u32x4 q = {0u, 0u, 0u, 0u};
-      if (i0 + 4 * j < hi) q = *reinterpret_cast<const u32x4*>(packed + i0 + 4 * j);
+      if (o0 + 4 * j < len) q = *reinterpret_cast<const u32x4*>(packed + base + (o0 + 4 * j));
       x[4 * j] = q.x;
       x[4 * j + 1] = q.y;
       x[4 * j + 2] = q.z;
@@ -1948,9 +1946,9 @@ __global__ void __launch_bounds__(kSortBlock) k_bin_sort(const uint32_t* __restr
     }
 #pragma unroll
     for (uint32_t b = 0; b < kSortBins; b += kSortBlock) s_bin[b + t] = 0;
-    const uint32_t first = max(i0, lo);
     uint32_t g = g0, end = 0;
-    if (first < hi) {
+    if (o0 < len) {
+      const uint32_t first = max(base + o0, lo);
       uint32_t z = g1 - 1;  // the last segment that begins at or before the first edge
       while (g < z) {
         const uint32_t mid = g + (z - g + 1) / 2;
@@ -1961,9 +1959,9 @@ __global__ void __launch_bounds__(kSortBlock) k_bin_sort(const uint32_t* __restr
     __syncthreads();
 #pragma unroll
     for (int j = 0; j < kSortPer; ++j) {
-      const uint32_t e = i0 + j;
       at[j] = INF32;
-      if (e < lo || e >= hi) continue;
+      if (o0 + j < lo - base || o0 + j >= len) continue;
+      const uint32_t e = base + o0 + j;
       while (end <= e) end = F2[++g + 1];
       const uint32_t bits = g < J * kHotSubs ? wl - kHotBits : wl;  // a segment's slots
       const uint32_t slot = x[j] & ((1u << bits) - 1u);
@@ -1996,7 +1994,7 @@ __global__ void __launch_bounds__(kSortBlock) k_bin_sort(const uint32_t* __restr
 }
 
 static void bin_sort(suminc_ctx* c, BinLayout& L, uint32_t J, uint32_t nseg, uint32_t m, uint32_t wl) {
-  const uint32_t tiles = (m + kSortStep - 1) / kSortStep;
+  const uint32_t tiles = sort_tiles(m);
   L.seg0.ensure_slack(((size_t)tiles + 1) * 4);
   k_bin_sort_tiles<<<grid_for((uint64_t)tiles + 1), kBlock, 0, c->stream>>>(L.F2.as<uint32_t>(), nseg, tiles,
                                                                            L.seg0.as<uint32_t>());
