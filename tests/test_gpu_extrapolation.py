@@ -379,15 +379,25 @@ def test_reseed_of_sources_that_gain_many_edges(gpu, prec, div):
     assert np.abs(d1 - want).sum() <= eps * 3 * (2 * sent + np.abs(d).sum() + np.abs(want).sum())
 
 
-@pytest.mark.parametrize("n,m", [(3000, 16383), (3000, 16384), (3000, 16385), (9000, 49157), (200_000, 100_000),
-                                 (200_000, 400_000)])
+@pytest.mark.parametrize("n,m,hot", [(3000, 16383, 0), (3000, 16384, 0), (3000, 16385, 0), (9000, 49157, 0),
+                                     (200_000, 100_000, 0), (200_000, 400_000, 0), (5000, 70_001, 8),
+                                     (4200, 90_000, 5)])
 @pytest.mark.parametrize("prec", ["fp64", "fp32"])
-def test_binned_layout_at_the_edges_of_its_sort_tiles(gpu, n, m, prec):
+def test_binned_layout_at_the_edges_of_its_sort_tiles(gpu, n, m, hot, prec):
     """The binned pull (1 KiB windows) with layouts around whole steps of the ordering
-    (8192 edges), a few segments a workgroup and more than its 4096 counters."""
+    (8192 edges), a few segments a workgroup and more than its 4096 counters; with `hot`
+    sources that reach every vertex, in the hottest range of slots (8), so that a block of
+    4096 destinations has a segment of 4096 * hot edges, beyond a chunk (16380)."""
     rng = np.random.default_rng(m)
     key = np.unique((n * rng.random(2 * m) ** 3).astype(np.int64) * n + (n * rng.random(2 * m) ** 2).astype(np.int64))
     key = key[key // n != key % n]
+    if hot:
+        row = (n * rng.random(m) ** 2).astype(np.int64) % (n - hot) + hot  # the others stay far below n out-edges
+        key = np.unique(row * n + rng.integers(0, n, m))
+        key = key[key // n != key % n]
+        all_of = np.arange(hot * n)
+        all_of = all_of[all_of // n != all_of % n]
+        key = np.concatenate([all_of, rng.permutation(key)[: m - len(all_of)]])
     key = np.sort(rng.permutation(key)[:m])
     assert len(key) == m
     u, v = key // n, key % n
@@ -404,7 +414,7 @@ def test_binned_layout_at_the_edges_of_its_sort_tiles(gpu, n, m, prec):
     with gpu.Context(pr_precision=p, termcheck_threshold=T, max_rounds=1000, pull_bin_kib=1) as ctx:
         ctx.upload_csr(off, v.astype(np.uint32), w)
         ctx.pr_init()
-        ctx.pr_run()
+        assert ctx.pr_run()["pull_rounds"] > 0
         r, _ = ctx.pr_download()
         ctx.wpr_set_weights(w)
         rw, _ = ctx.wpr_forward(x)
