@@ -476,9 +476,11 @@ int suminc_compress_mirror_load(suminc_ctx* ctx, const char* path, suminc_compre
  * termcheck_threshold.  Backward for L = sum_i c_i r_i: the same series on the
  * transpose graph from mu_0 = c, stopped when sum|mu| < termcheck_threshold * sum|c|,
  * gives lambda; dL/dp = (1-d) lambda, dL/dw_uv = (d r_u / s_u)(lambda_v - sum_k W[u,k]
- * lambda_k).  A series may take extrapolation steps, as suminc_pr_run does.  State in FP32 with Kahan sums or FP64 (pr_precision).  Vectors are n
- * floats, edge weights and their gradient m floats in out-CSR order; every pointer
- * may be host or device memory of the context's GPU.  All four synchronise.
+ * lambda_k).  A series may take extrapolation steps, as suminc_pr_run does.  State in
+ * FP32 with Kahan sums or FP64 (pr_precision).  Vectors are n floats, edge weights and
+ * their gradient m floats in out-CSR order; every pointer may be host or device memory
+ * of the context's GPU.  All four synchronise.  A forward or backward that fails leaves
+ * the caller's result arrays as they were (suminc_wpr_forward_noalloc does not).
  * suminc_wpr_backward differentiates the context's last forward (its rank and
  * weights); a caller that runs several forwards before their backwards runs the
  * forward again first (SUMINC_E_STATE when the weights or the graph changed since). */

@@ -836,12 +836,12 @@ static SeriesBufs<T> series_state(suminc_ctx* c, WprState& S, bool compact) {
 // Runs sum = sum_t x_t with x_{t+1} = A x_t from x_0 = scale * seed until
 // sum|x| < tol.  A's coefficients: a in the order of R's rows, a_csr in the CSR's (the
 // binned rounds).  Result (FP64) in out64, optionally FP32 in out32 (either may be
-// null).  pos != nullptr: R's columns are compact positions, and the rounds
+// null); a series that fails leaves out32 alone unless out32_always.  pos != nullptr: R's columns are compact positions, and the rounds
 // gather the compact copy of x (B.xc).  Allocates nothing itself.
 template <class T>
 static void wpr_series(suminc_ctx* c, const SeriesBufs<T>& B, const RowLists& R, const BinLayout* L,
                        const uint32_t* pos, const T* a, const T* a_csr, const float* seed_dev, T scale, double tol_abs, bool relative,
-                       float* out32, double* out64, suminc_stats* st) {
+                       float* out32, double* out64, suminc_stats* st, bool out32_always = false) {
   const uint32_t n = c->n;
   // the binned layout of R's direction when it exists: its coefficients taken in layout
   // order, the rounds through the gather and summing passes
@@ -873,16 +873,17 @@ static void wpr_series(suminc_ctx* c, const SeriesBufs<T>& B, const RowLists& R,
     if (c->host_counters->done) break;
     group = enqueued < 24 ? 4 : std::min(64, 2 * group);
   }
+  const Counters* h = c->host_counters;
+  const bool capped = h->residual >= h->dpad[0];
+  if ((h->aux[0] || capped) && !out32_always) out32 = nullptr;
   k_wpr_finish<T><<<g, kBlock, 0, c->stream>>>(n, B.x, B.y, B.sum, B.comp, cnt, out32, out64);
   SUMINC_HIP(hipGetLastError());
   SUMINC_HIP(hipEventRecord(c->ev_stop, c->stream));
   SUMINC_HIP(hipEventSynchronize(c->ev_stop));
   float ms = 0;
   SUMINC_HIP(hipEventElapsedTime(&ms, c->ev_start, c->ev_stop));
-  const Counters* h = c->host_counters;
   SUMINC_REQUIRE(!h->aux[0], SUMINC_E_NUMERIC, "NaN/Inf in the weighted PageRank state");
-  SUMINC_REQUIRE(!(h->residual >= h->dpad[0]), SUMINC_E_NOT_CONVERGED,
-                 "round cap reached before sum|delta| < tolerance");
+  SUMINC_REQUIRE(!capped, SUMINC_E_NOT_CONVERGED, "round cap reached before sum|delta| < tolerance");
   suminc_stats out{};
   out.rounds = (double)h->rounds;
   out.edges_traversed = (double)h->edges;
@@ -1139,7 +1140,7 @@ static void wpr_forward_noalloc_t(suminc_ctx* c, const float* p, float* r, sumin
   const uint32_t* pos = compact ? S.in.pos.as<uint32_t>() : nullptr;
   S.fwd_ready = false;  // the rank of this forward is not kept for a backward
   wpr_series<T>(c, B, R, &S.bin_in, pos, S.a_in.as<T>(), S.a_out.as<T>(), p, (T)(1.0 - c->prm.damping),
-                c->prm.termcheck_threshold, false, r, nullptr, st);
+                c->prm.termcheck_threshold, false, r, nullptr, st, true);
   SUMINC_HIP(hipStreamSynchronize(c->stream));
 }
 

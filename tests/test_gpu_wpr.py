@@ -199,3 +199,31 @@ def test_edge_passes_at_their_edges(gpu, case, bin_kib):
     for x, y in ((same[2], got), (same[3], gp), (same[4], gw)):
         assert np.abs(x - y).max() <= 2e-7 * np.abs(y).max() + zero
     assert np.array_equal(same[0], p) and np.array_equal(same[1], c)
+
+
+@pytest.mark.parametrize("where", ["device", "host"])
+def test_failed_series_leave_the_results_alone(gpu, where):
+    """A capped or NaN forward and a capped backward raise and do not write the caller's
+    arrays, in device memory as in host memory."""
+    g, off, col, w, p, c, _ = problem(10)
+    with gpu.Context(termcheck_threshold=1e-12, max_rounds=3) as ctx:
+        ctx.upload_csr(off, col, w)
+        put = ctx.device_array if where == "device" else (lambda x: x.copy())
+        get = (lambda x: x.download()) if where == "device" else (lambda x: x)
+        mark = np.full(g.n, -7.0, np.float32)
+        r, gp, gw = put(mark), put(mark), put(np.full(len(w), -7.0, np.float32))
+        with pytest.raises(gpu.SumincError) as e:
+            ctx.wpr_forward(put(p), out=r)
+        assert e.value.code == gpu.E_NOT_CONVERGED and (get(r) == -7).all()
+        bad = p.copy()
+        bad[5] = np.nan
+        with pytest.raises(gpu.SumincError) as e:
+            ctx.wpr_forward(put(bad), out=r)
+        assert e.value.code == gpu.E_NUMERIC and (get(r) == -7).all()
+        ctx.set_params(max_rounds=1000)
+        ctx.wpr_forward(put(p), out=r)
+        assert (get(r) != -7).all()
+        ctx.set_params(max_rounds=3)
+        with pytest.raises(gpu.SumincError) as e:
+            ctx.wpr_backward(put(c), grad_p=gp, grad_w=gw)
+        assert e.value.code == gpu.E_NOT_CONVERGED and (get(gp) == -7).all() and (get(gw) == -7).all()
