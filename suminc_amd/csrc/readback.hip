@@ -10,20 +10,15 @@
 // 2.5 -> 0.95 ms; 1000 vertices: 84 -> 50 us (no allocation).
 #include "readback.hpp"
 
-#include <atomic>
 #include <mutex>
-#include <system_error>
-#include <thread>
+#include <utility>
+
+#include "copiers.hpp"
 
 namespace suminc {
 
 namespace {
 
-// A chunk is large enough to amortise its launch and event (2 MiB cross in 40 us) and
-// small enough that every copying thread has one.
-constexpr size_t kChunkBytes = size_t(2) << 20;
-constexpr int kThreads = 8;
-constexpr int kSlots = 2 * kThreads;
 // Below this the calling thread copies alone: starting the threads costs 0.1 ms.
 constexpr size_t kThreadedBytes = size_t(4) << 20;
 
@@ -42,18 +37,14 @@ struct Ring {
 // gives it back; at most kIdle stay, none after the last context is gone.
 constexpr size_t kIdle = 2;
 std::mutex g_mu;
-std::vector<Ring*> g_idle;
+Ring* g_idle[kIdle] = {};
 size_t g_contexts = 0;
 
 Ring* ring_take(int device) {
   {
     std::lock_guard<std::mutex> lk(g_mu);
-    for (size_t i = 0; i < g_idle.size(); ++i)
-      if (g_idle[i]->device == device) {
-        Ring* r = g_idle[i];
-        g_idle.erase(g_idle.begin() + i);
-        return r;
-      }
+    for (Ring*& slot : g_idle)
+      if (slot && slot->device == device) return std::exchange(slot, nullptr);
   }
   Ring* r = new (std::nothrow) Ring();
   if (!r) return nullptr;
@@ -73,79 +64,23 @@ Ring* ring_take(int device) {
 void ring_give(Ring* r) {
   {
     std::lock_guard<std::mutex> lk(g_mu);
-    if (g_contexts && g_idle.size() < kIdle) {
-      g_idle.push_back(r);
-      return;
-    }
+    for (Ring*& slot : g_idle)
+      if (g_contexts && !slot) {
+        slot = r;
+        return;
+      }
   }
   delete r;
 }
 
-// Copies chunks [0, n) as they become ready; chunk i is thread i % threads' (the calling
-// thread's own, as the last step of post(), without threads).
-struct Copiers {
-  const std::vector<Chunk>& chunks;
-  Ring* ring;
-  std::atomic<size_t> ready{0};
-  std::atomic<bool> stop{false};
-  std::vector<std::atomic<size_t>> done;  // per slot: chunks copied out of it
-  std::vector<std::thread> threads;
-
-  Copiers(const std::vector<Chunk>& c, Ring* r, bool threaded) : chunks(c), ring(r), done(kSlots) {
-    if (!threaded) return;
-    const unsigned hw = std::thread::hardware_concurrency();
-    const int want = (int)std::min<size_t>(std::min<unsigned>(kThreads, hw ? hw : 1u), chunks.size());
-    try {
-      threads.reserve(want);
-      for (int t = 0; t < want; ++t) threads.emplace_back([this, t, want] { work(t, want); });
-    } catch (const std::system_error&) {  // no threads to be had: the calling thread copies
-      stop_all();
-      threads.clear();
-      stop = false;
-    }
-  }
-  ~Copiers() { stop_all(); }
-  void stop_all() {
-    stop = true;
-    for (std::thread& t : threads)
-      if (t.joinable()) t.join();
-  }
-  void copy(size_t i) {
-    const Chunk& k = chunks[i];
-    std::memcpy(k.dst, ring->mem + (i % kSlots) * kChunkBytes, k.bytes);
-    done[i % kSlots].fetch_add(1, std::memory_order_release);
-  }
-  void work(size_t t, size_t step) {
-    for (size_t i = t; i < chunks.size(); i += step) {
-      while (ready.load(std::memory_order_acquire) <= i) {
-        if (stop.load(std::memory_order_relaxed)) return;
-        std::this_thread::yield();
-      }
-      copy(i);
-    }
-  }
-  void post(size_t i) {
-    if (threads.empty()) copy(i);
-    else ready.store(i + 1, std::memory_order_release);
-  }
-  void wait_free(size_t i) {  // slot of chunk i is free: every earlier chunk in it was copied
-    while (done[i % kSlots].load(std::memory_order_acquire) < i / kSlots) std::this_thread::yield();
-  }
-  void finish() {
-    const size_t n = chunks.size();
-    for (size_t s = 0; s < kSlots && s < n; ++s)
-      while (done[s].load(std::memory_order_acquire) < (n - s + kSlots - 1) / kSlots) std::this_thread::yield();
-  }
-};
-
 }  // namespace
 
 void readback_context(int change) {
-  std::vector<Ring*> gone;
+  Ring* gone[kIdle] = {};
   {
     std::lock_guard<std::mutex> lk(g_mu);
     g_contexts += change;
-    if (!g_contexts) gone.swap(g_idle);
+    if (!g_contexts) std::swap(gone, g_idle);
   }
   for (Ring* r : gone) delete r;
 }
@@ -185,7 +120,7 @@ bool readback(suminc_ctx* c, const std::vector<ReadbackPart>& parts, const Readb
     hipStream_t s;
     ~Drain() { (void)hipStreamSynchronize(s); }
   } drain{c->stream};
-  Copiers copiers(chunks, ring, total >= kThreadedBytes);
+  Copiers copiers(chunks, ring->mem, total >= kThreadedBytes);
   const size_t n = chunks.size();
   size_t sent = 0;
   for (size_t i = 0; i < n; ++i) {

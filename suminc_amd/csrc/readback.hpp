@@ -13,12 +13,6 @@ struct ReadbackPart {
   uint64_t count;
   size_t elem;
 };
-struct Chunk {
-  int part;
-  uint64_t first, count;
-  unsigned char* dst;
-  size_t bytes;
-};
 // Enqueues on the context's stream the kernel that stores elements
 // [first, first + count) of a part at out (pinned memory).
 using ReadbackLaunch = std::function<void(int part, uint64_t first, uint64_t count, void* out)>;
