@@ -49,7 +49,7 @@
 
 namespace suminc {
 
-constexpr int kCountPer = 4;  // vertices per thread of k_pr_count and k_pr_gather
+constexpr int kCountPer = kVertexPer;  // vertices per thread of k_pr_count and k_pr_gather
 
 // Block sums of the round: FP64 partials of gridDim.x values each, sum |delta| at 0,
 // the active vertices' out-degrees (u64) at 1, and with a candidate extrapolation
@@ -822,7 +822,7 @@ void pr_alloc(suminc_ctx* c) {
   c->wl1.ensure(n * es + 8);
   // heavy chunks: at most m / kChunk + (number of heavy vertices) entries
   c->heavy.ensure_slack((c->m / kChunk + c->m / kHeavyDeg + 2) * sizeof(uint4));
-  c->partial.ensure(((size_t)grid_for(n) + 1) * 3 * 8);  // residual | edges | active vertices
+  c->partial.ensure(round_partials(c->n) * 8);
   c->tmp4.ensure(65536);  // per-round scatter mode history
 }
 

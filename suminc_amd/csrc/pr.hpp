@@ -19,6 +19,11 @@ void pr_step(suminc_ctx* c, double* residual);
 void pr_download(suminc_ctx* c, double* rank, double* delta);
 void pr_upload(suminc_ctx* c, const double* rank, const double* delta);
 unsigned push_grid();
+// Vertices per thread of the rounds' vertex passes, and the FP64 block sums (c->partial)
+// that a round leaves: five arrays of one value per workgroup of these passes, and in a
+// sketch round one value per workgroup of the pass over the exits (at most n of them).
+constexpr int kVertexPer = 4;
+inline size_t round_partials(uint32_t n) { return (size_t)5 * grid_for(n, kBlock * kVertexPer) + grid_for(n); }
 // clears the device counters on the stream (the start of a run)
 void zero_counters(suminc_ctx* c);
 // positions of the vertices by decreasing degree (deg_off's row lengths; degree 0:

@@ -1413,7 +1413,7 @@ struct SkArgs {
 // sums in arrays of gridDim.x: the residual at 0, the edges (u64) at 1, and with a
 // candidate extrapolation (cnt->ex.cand > 0) the same of the extrapolated state at 2
 // and 3.  kSkPer vertices a thread (vertex base + j * kBlock + t, coalesced).
-constexpr int kSkPer = 4;
+constexpr int kSkPer = kVertexPer;
 template <class T>
 __global__ void __launch_bounds__(kBlock) k_sk_count(SkArgs a, const T* __restrict__ delta,
                                                      const T* __restrict__ prev, const T* __restrict__ bound,

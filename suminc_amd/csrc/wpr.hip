@@ -783,8 +783,9 @@ struct SeriesBufs {
   double *partial, *l1;
 };
 
-// Bytes of the series buffers for n vertices (partials: one per vertex block, three
-// words each, as the PageRank rounds size them).
+// Bytes of the series buffers for n vertices (partials: the seed pass leaves one value per
+// vertex block, the count two per workgroup of kStepPer vertices a thread: room for three
+// per vertex block, which also fixes the largest n that the scratch array takes).
 template <class T>
 static size_t series_bytes(uint32_t n, bool compact) {
   auto al = [](size_t b) { return (b + 255) & ~size_t(255); };
