@@ -272,6 +272,7 @@ struct suminc_ctx {
 
   // rounds enqueued before the first host check (last run's rounds + 1)
   int hint_reset = 6, hint_sssp = 8, hint_sssp_sketch = 8;
+  bool hint_sssp_push = false;  // the last traversal from scratch that could pull did not
 
   // weighted PageRank / adjoint state (wpr.hip), created on first use
   void* wpr = nullptr;

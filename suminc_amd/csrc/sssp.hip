@@ -141,6 +141,13 @@ __global__ void __launch_bounds__(kBlock) k_sssp_heavy(SsspArgs a) {
 // ---- pull rounds --------------------------------------------------------------------
 constexpr uint32_t kPullTile = 1024;     // CSC edges per workgroup
 constexpr uint32_t kPullFrontier = 64;   // a pull from n / 64 frontier vertices on
+// Rounds are enqueued without the pull's launches after a group of rounds that had no pull
+// and left a frontier below n / 256, and from the start where the last run from scratch
+// had none.  Long paths and road graphs are such runs: two of their five launches a round
+// return at once (BFS of 4999 rounds on a 2500 x 2500 grid: 193 ms with them, 154 without;
+// of 20,000 rounds on a path of a graph of 340,000 edges: 249 and 198).  A frontier that
+// grows past n / 64 all the same stops the group (k_sssp_end).
+constexpr uint32_t kPushFrontier = 256;
 constexpr uint64_t kPullMinEdges = 1u << 18;  // below, a push round costs less than the further launches
 
 struct SsspPull {
@@ -377,7 +384,10 @@ __global__ void __launch_bounds__(1024) k_sssp_turn(Counters* cnt, uint32_t n, c
   if (cnt->wl_count[nxt] == 0 || (long long)cnt->rounds >= (long long)max_rounds) cnt->done = 1;
 }
 
-__global__ void k_sssp_end(Counters* cnt, int max_rounds) {
+// Closes a push round.  n_pull (0: no pulls): the vertices of a run that may pull but whose
+// rounds are enqueued without it; a frontier to pull from stops the group, and the first
+// round of the next one is a pull that passes over no row for its word (cnt->rc).
+__global__ void k_sssp_end(Counters* cnt, int max_rounds, uint32_t n_pull) {
   if (threadIdx.x != 0 || cnt->done) return;
   const int cur = (int)(cnt->aux[1] & 1), nxt = cur ^ 1;
   cnt->aux[6] += cnt->wl_count[cur];  // frontier vertices processed
@@ -385,7 +395,17 @@ __global__ void k_sssp_end(Counters* cnt, int max_rounds) {
   cnt->heavy_count = 0;
   cnt->rounds += 1;
   cnt->aux[1] ^= 1ull;
-  if (cnt->wl_count[nxt] == 0 || (long long)cnt->rounds >= (long long)max_rounds) cnt->done = 1;
+  if (cnt->wl_count[nxt] == 0 || (long long)cnt->rounds >= (long long)max_rounds) {
+    cnt->done = 1;
+  } else if (n_pull && cnt->wl_count[nxt] * kPullFrontier > n_pull) {
+    cnt->mode = 1;
+    cnt->rc[nxt] = 0;
+    cnt->done = 1;
+  }
+}
+
+__global__ void k_sssp_resume(Counters* cnt) {
+  if (threadIdx.x == 0) cnt->done = 0;
 }
 
 __global__ void k_sssp_init(uint32_t n, unsigned long long* dp, uint32_t src) {
@@ -511,25 +531,39 @@ void sssp_run(suminc_ctx* c, suminc_stats* st) {
                                                                          c->sssp_tile.as<uint32_t>());
   k_sssp_begin<<<1, 64, 0, c->stream>>>(a.cnt, c->sssp_seeds.as<unsigned long long>());
   int group = c->hint_sssp;  // rounds of the previous query + 1 first
+  bool pulling = pulls && !c->hint_sssp_push;  // this group's rounds may pull
+  unsigned long long pulled = 0;
   size_t slot = 0;
   while (true) {
     for (int i = 0; i < group; ++i, ++slot) {
       if (c->prof_on) SUMINC_HIP(hipEventRecord(prof_event(c, 2 * slot), c->stream));
       k_sssp_push<<<push_grid(), kBlock, 0, c->stream>>>(a);
       k_sssp_heavy<<<push_grid(), kBlock, 0, c->stream>>>(a);
-      if (pulls) k_sssp_pull<<<tiles, kBlock, 0, c->stream>>>(a, p);
+      if (pulling) k_sssp_pull<<<tiles, kBlock, 0, c->stream>>>(a, p);
       if (c->prof_on) SUMINC_HIP(hipEventRecord(prof_event(c, 2 * slot + 1), c->stream));
-      if (pulls) {
+      if (pulling) {
         k_sssp_collect<<<grid_for((c->n + 31) / 32), kBlock, 0, c->stream>>>(a, c->n);
         k_sssp_turn<<<1, 1024, 0, c->stream>>>(a.cnt, c->n, p.edges, tiles, max_rounds);
       } else {
-        k_sssp_end<<<1, 64, 0, c->stream>>>(a.cnt, max_rounds);
+        k_sssp_end<<<1, 64, 0, c->stream>>>(a.cnt, max_rounds, pulls ? c->n : 0u);
       }
     }
     SUMINC_HIP(hipGetLastError());
     read_counters(c);
-    if (c->host_counters->done) break;
+    const Counters* h = c->host_counters;
+    const unsigned long long front = h->wl_count[h->aux[1] & 1];
+    if (h->done) {
+      if (pulling || !pulls || front == 0 || h->rounds >= (unsigned long long)max_rounds) break;
+      // stopped for its frontier: the group's other rounds did nothing
+      k_sssp_resume<<<1, 64, 0, c->stream>>>(a.cnt);
+      slot = (size_t)h->rounds;
+      group = 8;
+      pulling = true;
+      continue;
+    }
     if (group < 64) group *= 2;
+    pulling = pulls && (h->mode != 0 || h->pull_rounds != pulled || front * kPushFrontier > c->n);
+    pulled = h->pull_rounds;
   }
   SUMINC_HIP(hipEventRecord(c->ev_stop, c->stream));
   SUMINC_HIP(hipEventSynchronize(c->ev_stop));
@@ -537,6 +571,7 @@ void sssp_run(suminc_ctx* c, suminc_stats* st) {
   SUMINC_HIP(hipEventElapsedTime(&ms, c->ev_start, c->ev_stop));
   Counters* h = c->host_counters;
   c->hint_sssp = std::max(2, std::min(64, (int)h->rounds + 1));
+  if (pulls) c->hint_sssp_push = h->pull_rounds == 0;
   if (c->prof_on) {
     prof_collect(c, SUMINC_KERNEL_SSSP_PUSH, (size_t)h->rounds, 0, 2);
     suminc_kernel_profile& p = c->prof[SUMINC_KERNEL_SSSP_PUSH];
@@ -582,7 +617,7 @@ void sssp_step(suminc_ctx* c, uint32_t* frontier_out) {
   k_sssp_begin<<<1, 64, 0, c->stream>>>(a.cnt, c->sssp_seeds.as<unsigned long long>());
   k_sssp_push<<<push_grid(), kBlock, 0, c->stream>>>(a);
   k_sssp_heavy<<<push_grid(), kBlock, 0, c->stream>>>(a);
-  k_sssp_end<<<1, 64, 0, c->stream>>>(a.cnt, 1 << 30);
+  k_sssp_end<<<1, 64, 0, c->stream>>>(a.cnt, 1 << 30, 0);
   k_sssp_carry<<<1, 64, 0, c->stream>>>(a.cnt, c->sssp_seeds.as<unsigned long long>());
   SUMINC_HIP(hipGetLastError());
   read_counters(c);

@@ -1,8 +1,9 @@
 """Traversals whose rounds pull (a run from scratch on 2^18 edges or more): SSSP and BFS
 equal the unique fixed point bit for bit, distances and smallest-id parents; SSWP widths
 equal it and its parents are valid and acyclic.  Graphs: R-MAT, rows across many 1024-edge
-tiles, tiles that run over tens of thousands of empty rows (the per-edge search), and a
-frontier that grows and shrinks around the switch between push and pull."""
+tiles, tiles that run over tens of thousands of empty rows (the per-edge search), a
+frontier that grows and shrinks around the switch between push and pull, and one that
+stays small for longer than the first group of rounds."""
 import numpy as np
 import pytest
 
@@ -37,6 +38,10 @@ def graph(name, rng):
         ends = np.concatenate([np.arange(0, 3000), np.arange(n - 3000, n)])
         u, v = rng.choice(ends, 330_000), rng.choice(ends, 330_000)
         u[:300], v[:300] = 0, rng.choice(ends, 300)
+    elif name == "late":  # a path of 150 into a core: rounds enqueued without pulls meet the core's frontier
+        n = 30_150
+        core = 150 + rng.integers(0, n - 150, (2, 300_000))
+        u, v = np.concatenate([np.arange(150), core[0]]), np.concatenate([np.arange(1, 151), core[1]])
     else:  # layers: 5 vertices, then 200, 20,000, 20,000, 50, 20,000, 10
         sizes = [1, 5, 200, 20_000, 20_000, 50, 20_000, 10]
         n = sum(sizes)
@@ -69,7 +74,7 @@ def relax(n, u, v, w, app):
 
 
 @pytest.mark.parametrize("app", ["sssp", "bfs", "sswp"])
-@pytest.mark.parametrize("name", ["rmat", "hubs", "gaps", "layers"])
+@pytest.mark.parametrize("name", ["rmat", "hubs", "gaps", "late", "layers"])
 def test_pull_rounds_reach_the_fixed_point(gpu, name, app):
     n, off, col, w, u, v = graph(name, np.random.default_rng(4))
     assert len(col) >= 1 << 18
@@ -108,6 +113,44 @@ def test_pull_rounds_reach_the_fixed_point(gpu, name, app):
     for _ in range(int(n).bit_length()):
         up = up[up]
     assert (up[reached] == 0).all()
+
+
+@pytest.mark.parametrize("app", ["sssp", "bfs"])
+def test_a_run_without_pulls_before_one_with_them(gpu, app):
+    """After a run from scratch that had no pull, the next one's rounds are enqueued
+    without, until its frontier asks for one; at a round cap on either side of that too."""
+    n, off, col, w, u, v = graph("late", np.random.default_rng(6))
+    code = {"sssp": gpu.APP_SSSP, "bfs": gpu.APP_BFS}[app]
+    with gpu.Context() as ctx:
+        ctx.upload_csr(off, col, w)
+
+        def run(source, cap=0):
+            ctx.set_params(max_rounds=cap or 100000)
+            ctx.traversal_init(code, source)
+            try:
+                st = ctx.sssp_run()
+            except gpu.SumincError as e:
+                assert e.code == gpu.E_NOT_CONVERGED
+                st = ctx.stats()
+            return st, *ctx.sssp_download()
+
+        first = run(150)
+        assert first[0]["pull_rounds"] > 0
+        ctx.set_params(max_rounds=20)
+        caps = {}
+        for cap in (1, 2, 3, 4, 5, 7):
+            caps[cap] = run(150, cap)
+        for cap in caps:
+            assert run(0, 40)[0]["pull_rounds"] == 0  # on the path only: no pull
+            st, val, par = run(150, cap)
+            assert st["rounds"] == min(cap, first[0]["rounds"])
+            # (a capped SSSP's words depend on the order of the round; BFS' do not)
+            if app == "bfs":
+                assert np.array_equal(val, caps[cap][1])
+            assert run(0, 40)[0]["pull_rounds"] == 0
+            st, val, par = run(150)
+            assert st["pull_rounds"] > 0 and st["pull_rounds"] + st["push_rounds"] == st["rounds"]
+            assert np.array_equal(val, first[1]) and np.array_equal(par, first[2])
 
 
 def test_widths_with_many_ties_keep_a_tree_of_parents(gpu):
