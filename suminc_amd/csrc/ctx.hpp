@@ -273,6 +273,8 @@ struct suminc_ctx {
   // rounds enqueued before the first host check (last run's rounds + 1)
   int hint_reset = 6, hint_sssp = 8, hint_sssp_sketch = 8;
   bool hint_sssp_push = false;  // the last traversal from scratch that could pull did not
+  // the same of PageRank runs: plain, the plain rounds behind a sketch phase, sketch
+  int hint_pr = 10, hint_pr_rest = 4, hint_sk = 10;
 
   // weighted PageRank / adjoint state (wpr.hip), created on first use
   void* wpr = nullptr;

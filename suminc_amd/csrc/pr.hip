@@ -822,6 +822,7 @@ void pr_alloc(suminc_ctx* c) {
   c->wl1.ensure(n * es + 8);
   // heavy chunks: at most m / kChunk + (number of heavy vertices) entries
   c->heavy.ensure_slack((c->m / kChunk + c->m / kHeavyDeg + 2) * sizeof(uint4));
+  c->hint_pr = c->hint_sk = 10;  // a run from a new state
   c->partial.ensure(round_partials(c->n) * 8);
   c->tmp4.ensure(65536);  // per-round scatter mode history
 }
@@ -2365,7 +2366,7 @@ static void enqueue_tiny(suminc_ctx* c, double eps, double T_stop, int max_round
 }
 
 // Runs rounds until the device sets the stop flag; host polls every `group` rounds.
-void pr_run(suminc_ctx* c, suminc_stats* st) {
+void pr_run(suminc_ctx* c, suminc_stats* st, bool rest) {
   SUMINC_REQUIRE(c->pr_ready, SUMINC_E_STATE, "PageRank state not initialised");
   const double T = c->prm.termcheck_threshold;
   const double eps = T / (double)c->n;
@@ -2374,8 +2375,8 @@ void pr_run(suminc_ctx* c, suminc_stats* st) {
   if (div > 0 && !(c->n <= kTinyN && c->m <= kTinyM && !c->prof_on)) ensure_pull_heavy(c);
   zero_counters(c);
   SUMINC_HIP(hipEventRecord(c->ev_start, c->stream));
-  // extrapolated runs take 8-16 rounds; one poll costs about as much as three empty rounds
-  int group = 10;
+  int& hint = rest ? c->hint_pr_rest : c->hint_pr;
+  int group = hint;
   size_t slot = 0;
   const bool tiny = c->n <= kTinyN && c->m <= kTinyM && !c->prof_on;  // the profile times single launches
   while (true) {
@@ -2393,11 +2394,12 @@ void pr_run(suminc_ctx* c, suminc_stats* st) {
     SUMINC_HIP(hipEventRecord(c->ev_stop, c->stream));
     read_counters(c);
     if (c->host_counters->done) break;
-    group = slot < 20 ? 4 : std::min(32, 2 * group);
+    group = next_group(group, slot);
   }
   float ms = 0;
   SUMINC_HIP(hipEventElapsedTime(&ms, c->ev_start, c->ev_stop));
   Counters* h = c->host_counters;
+  hint = first_group((int)h->rounds);
   pr_profile_rounds(c, (size_t)h->rounds);
   c->stats = suminc_stats{};
   c->stats.rounds = (double)h->rounds;

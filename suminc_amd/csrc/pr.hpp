@@ -1,5 +1,6 @@
 // pr.hpp -- host-side entry points of the device algorithms (called by capi.hip).
 #pragma once
+#include <algorithm>
 #include "ctx.hpp"
 
 namespace suminc {
@@ -14,7 +15,17 @@ void download_csr(suminc_ctx* c, uint64_t* off, uint32_t* col, void* w, bool in_
 // pr.hip
 void pr_alloc(suminc_ctx* c);
 void pr_init(suminc_ctx* c);
-void pr_run(suminc_ctx* c, suminc_stats* st);
+// rest: the plain rounds that follow a sketch phase (few, if any)
+void pr_run(suminc_ctx* c, suminc_stats* st, bool rest = false);
+// Rounds to enqueue before the host looks at the counters.  Extrapolated runs from scratch
+// take 8-16 rounds, and a look costs about as much as three empty rounds; but a query on a
+// converged state has none or a few, so a run's first group is what the run before needed,
+// 4 to 10 (65,536 vertices, nothing to do: 192 us behind 10 rounds of launches, over the
+// sketch 561; behind 4 rounds 114 and 314).
+inline int first_group(int rounds) { return std::max(4, std::min(10, rounds + 1)); }
+inline int next_group(int group, size_t enqueued) {
+  return enqueued < 10 ? 10 - (int)enqueued : enqueued < 20 ? 4 : std::min(32, 2 * group);
+}
 void pr_step(suminc_ctx* c, double* residual);
 void pr_download(suminc_ctx* c, double* rank, double* delta);
 void pr_upload(suminc_ctx* c, const double* rank, const double* delta);

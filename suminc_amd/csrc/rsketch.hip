@@ -798,7 +798,7 @@ static void rsk_run_t(suminc_ctx* c, suminc_stats* st) {
   float ms_sketch = 0;
   SUMINC_HIP(hipEventElapsedTime(&ms_sketch, c->ev_start, c->ev_stop));
   suminc_stats rs{};
-  pr_run(c, &rs);  // the plain residual phase
+  pr_run(c, &rs, true);  // the plain residual phase
   suminc_stats out = rs;
   out.rounds = rs.rounds + rounds;
   out.kernel_ms = rs.kernel_ms + ms_sketch;

@@ -2081,7 +2081,7 @@ static void sum_pr_run_t(suminc_ctx* c, suminc_stats* st) {
   const unsigned ge = grid_for(n_exits);             // the exit pass
   c->tmp4.ensure(65536);  // per-round scatter mode (profile attribution)
   s.ex_taken.ensure(n_exits * es + es);
-  int group = 10;  // as the plain rounds
+  int group = c->hint_sk;
   size_t slot = 0;
   while (true) {
     for (int i = 0; i < group; ++i, ++slot) {
@@ -2112,9 +2112,10 @@ static void sum_pr_run_t(suminc_ctx* c, suminc_stats* st) {
     SUMINC_HIP(hipGetLastError());
     read_counters(c);
     if (c->host_counters->done) break;
-    group = slot < 20 ? 4 : std::min(32, 2 * group);
+    group = next_group(group, slot);
   }
   const Counters* h = c->host_counters;
+  c->hint_sk = first_group((int)h->rounds);
   out.sketch_rounds = (double)h->rounds;  // sketch rounds
   if (c->prof_on && h->rounds) {
     // the sketch rounds' pull launches (the plain rounds' kernel): device time of
@@ -2166,7 +2167,7 @@ static void sum_pr_run_t(suminc_ctx* c, suminc_stats* st) {
   const double sketch_edges = (double)h->edges;
   // 5. residual phase: plain Ingress rounds on the full graph
   suminc_stats rs{};
-  pr_run(c, &rs);
+  pr_run(c, &rs, true);
   out.rounds = rs.rounds + out.sketch_rounds;
   out.edges_traversed = rs.edges_traversed + sketch_edges + (double)wk;
   out.residual = rs.residual;

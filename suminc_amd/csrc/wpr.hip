@@ -609,6 +609,7 @@ struct WprState {
   uint64_t weights_version = 0;
   bool fwd_ready = false;
   uint64_t fwd_coef_version = ~0ull;
+  int hint_fwd = 12, hint_bwd = 12, hint_php = 12;  // rounds of the last run + 1: a series' first group
   WprDir out, in;
   DevBuf eid;                        // CSR edge id per CSC position
   DevBuf tile_row;                   // the row of the first edge of every edge tile of the CSR
@@ -837,10 +838,11 @@ static SeriesBufs<T> series_state(suminc_ctx* c, WprState& S, bool compact) {
 // Runs sum = sum_t x_t with x_{t+1} = A x_t from x_0 = scale * seed until
 // sum|x| < tol.  A's coefficients: a in the order of R's rows, a_csr in the CSR's (the
 // binned rounds).  Result (FP64) in out64, optionally FP32 in out32 (either may be
-// null); a series that fails leaves out32 alone unless out32_always.  pos != nullptr: R's columns are compact positions, and the rounds
+// null); a series that fails leaves out32 alone unless out32_always.  hint: the rounds to
+// enqueue first, then what the next run of this series is to.  pos != nullptr: R's columns are compact positions, and the rounds
 // gather the compact copy of x (B.xc).  Allocates nothing itself.
 template <class T>
-static void wpr_series(suminc_ctx* c, const SeriesBufs<T>& B, const RowLists& R, const BinLayout* L,
+static void wpr_series(suminc_ctx* c, int& hint, const SeriesBufs<T>& B, const RowLists& R, const BinLayout* L,
                        const uint32_t* pos, const T* a, const T* a_csr, const float* seed_dev, T scale, double tol_abs, bool relative,
                        float* out32, double* out64, suminc_stats* st, bool out32_always = false) {
   const uint32_t n = c->n;
@@ -859,8 +861,9 @@ static void wpr_series(suminc_ctx* c, const SeriesBufs<T>& B, const RowLists& R,
   k_wpr_start<<<1, 1024, 0, c->stream>>>(B.partial, g, B.l1, cnt);
   const int max_rounds = c->prm.max_rounds > 0 ? c->prm.max_rounds : 100000;
   SUMINC_HIP(hipEventRecord(c->ev_start, c->stream));
-  // extrapolated series take 9-20 rounds; one poll costs about as much as three empty rounds
-  int group = 12, enqueued = 0;
+  // extrapolated series take 9-20 rounds, others up to hundreds, loose tolerances one or
+  // two; a look at the counters costs about as much as three empty rounds
+  int group = hint, enqueued = 0;
   while (true) {
     for (int i = 0; i < group; ++i, ++enqueued) {
       if (binned) bin_layout_spmv<T, true>(c, *L, pos ? xc : B.x, B.y, cnt, 2);
@@ -872,9 +875,10 @@ static void wpr_series(suminc_ctx* c, const SeriesBufs<T>& B, const RowLists& R,
     SUMINC_HIP(hipGetLastError());
     read_counters(c);
     if (c->host_counters->done) break;
-    group = enqueued < 24 ? 4 : std::min(64, 2 * group);
+    group = enqueued < 12 ? 12 - enqueued : enqueued < 24 ? 4 : std::min(64, enqueued / 2);
   }
   const Counters* h = c->host_counters;
+  hint = std::max(4, std::min(64, (int)h->rounds + 1));
   const bool capped = h->residual >= h->dpad[0];
   if ((h->aux[0] || capped) && !out32_always) out32 = nullptr;
   k_wpr_finish<T><<<g, kBlock, 0, c->stream>>>(n, B.x, B.y, B.sum, B.comp, cnt, out32, out64);
@@ -966,7 +970,7 @@ static void wpr_forward_t(suminc_ctx* c, const float* p, float* r, suminc_stats*
   float* rd = r ? vector_out(c, r, n, S.out_f) : nullptr;
   const RowLists R = lists_of(S.in, c->in_off, c->in_col, true);
   const uint32_t* pos = S.in.compact ? S.in.pos.as<uint32_t>() : nullptr;
-  wpr_series<T>(c, series_state<T>(c, S, pos != nullptr), R, &S.bin_in, pos, S.a_in.as<T>(), S.a_out.as<T>(), pd,
+  wpr_series<T>(c, S.hint_fwd, series_state<T>(c, S, pos != nullptr), R, &S.bin_in, pos, S.a_in.as<T>(), S.a_out.as<T>(), pd,
                 (T)(1.0 - c->prm.damping), c->prm.termcheck_threshold, false, rd, S.r64.as<double>(), st);
   vector_home(c, r, rd, n);
   SUMINC_HIP(hipStreamSynchronize(c->stream));
@@ -987,7 +991,7 @@ static void wpr_backward_t(suminc_ctx* c, const float* cvec, float* grad_p, floa
   S.lam64.ensure((size_t)n * 8 + 8);
   const RowLists R = lists_of(S.out, c->out_off, c->out_col, true);
   const uint32_t* pos = S.out.compact ? S.out.pos.as<uint32_t>() : nullptr;
-  wpr_series<T>(c, series_state<T>(c, S, pos != nullptr), R, &S.bin_out, pos, S.a_out.as<T>(), S.a_out.as<T>(), cd,
+  wpr_series<T>(c, S.hint_bwd, series_state<T>(c, S, pos != nullptr), R, &S.bin_out, pos, S.a_out.as<T>(), S.a_out.as<T>(), cd,
                 (T)1, c->prm.termcheck_threshold, true, nullptr, S.lam64.as<double>(), st);
   const double* lam = S.lam64.as<double>();
   if (grad_p) {
@@ -1064,7 +1068,7 @@ static void php_run_t(suminc_ctx* c, uint32_t src, double d, double* values, sum
   SUMINC_HIP(hipGetLastError());
   const RowLists R = lists_of(S.in, c->in_off, c->in_col, true);
   const uint32_t* pos = S.in.compact ? S.in.pos.as<uint32_t>() : nullptr;
-  wpr_series<T>(c, series_state<T>(c, S, pos != nullptr), R, &S.bin_in, pos, S.php_a_in.as<T>(),
+  wpr_series<T>(c, S.hint_php, series_state<T>(c, S, pos != nullptr), R, &S.bin_in, pos, S.php_a_in.as<T>(),
                 S.php_a_out.as<T>(), S.in_f.as<float>(), (T)1, c->prm.termcheck_threshold, false, nullptr, S.php64.as<double>(), st);
   if (readback(c, {{values, n, 8}}, [c, &S](int, uint64_t first, uint64_t count, void* out) {
         k_copy_f64<<<grid_for(count), kBlock, 0, c->stream>>>((uint32_t)count, S.php64.as<double>() + first,
@@ -1140,7 +1144,7 @@ static void wpr_forward_noalloc_t(suminc_ctx* c, const float* p, float* r, sumin
   const RowLists R = lists_of(S.in, c->in_off, c->in_col, true);
   const uint32_t* pos = compact ? S.in.pos.as<uint32_t>() : nullptr;
   S.fwd_ready = false;  // the rank of this forward is not kept for a backward
-  wpr_series<T>(c, B, R, &S.bin_in, pos, S.a_in.as<T>(), S.a_out.as<T>(), p, (T)(1.0 - c->prm.damping),
+  wpr_series<T>(c, S.hint_fwd, B, R, &S.bin_in, pos, S.a_in.as<T>(), S.a_out.as<T>(), p, (T)(1.0 - c->prm.damping),
                 c->prm.termcheck_threshold, false, r, nullptr, st, true);
   SUMINC_HIP(hipStreamSynchronize(c->stream));
 }
