@@ -121,6 +121,7 @@ struct Counters {
   unsigned long long bcopy[4];      // a batch's group counts, copied out with the counters
   unsigned long long reseed_mode;   // PageRank reseed scatter: 0 push, 1 pull
   Extrap ex;                        // extrapolation of the running series
+  Extrap ex2[2];                    // the same by round parity (k_wpr_turn)
   unsigned long long pull_run;      // pull rounds in a row (sketch rounds)
 };
 

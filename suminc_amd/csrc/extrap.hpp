@@ -70,13 +70,14 @@ __device__ __forceinline__ void rank_add_wide(T* rank, float* comp, uint32_t v, 
 }
 
 // Sums of a block's values of each of the K arrays of nparts (double or u64 bits per
-// kU bit k) into out[K], in a fixed order; all threads of a 1024-thread block.
-template <int K, unsigned kU>
+// kU bit k) into out[K], in a fixed order; all threads of a block of kThreads.  Up to
+// kThreads parts the sums are the same for every kThreads.
+template <int K, unsigned kU, int kThreads = 1024>
 __device__ __forceinline__ void sum_parts(const double* __restrict__ partial, uint32_t nparts, double (*s)[K]) {
   double acc[K];
 #pragma unroll
   for (int k = 0; k < K; ++k) acc[k] = 0.0;  // the bits of u64 zero too
-  for (uint32_t i = threadIdx.x; i < nparts; i += 1024) {
+  for (uint32_t i = threadIdx.x; i < nparts; i += kThreads) {
 #pragma unroll
     for (int k = 0; k < K; ++k) {
       const double x = partial[(size_t)k * nparts + i];
@@ -103,7 +104,7 @@ __device__ __forceinline__ void sum_parts(const double* __restrict__ partial, ui
   }
   __syncthreads();
   if (threadIdx.x == 0) {
-    for (int w = 1; w < 1024 / 64; ++w) {
+    for (int w = 1; w < kThreads / 64; ++w) {
 #pragma unroll
       for (int k = 0; k < K; ++k) {
         if (kU >> k & 1)

@@ -143,8 +143,11 @@ __device__ __forceinline__ void kahan(T* sum, float* comp, uint32_t v, T x) {
 
 // A series' rounds: product, count, decision, step.  The decision comes before the
 // step, so that a step can be an extrapolation (extrap.hpp) at no further array: x and y
-// are its two points.  On R-MAT of 2^22 vertices, 50M edges, forward from 1024 seeds and
-// adjoint, both to 1e-9: 197 rounds, 51 ms -> 28 rounds, 8 ms.
+// are its two points.  Up to kBlock partials (2^18 vertices) every workgroup of the step
+// decides by itself (k_wpr_turn), which spares a launch of the four: the adjoint on a random
+// bipartite graph of 16,384 vertices, which never lines up, takes 59 rounds in 1.15 ms
+// (1.59 with a launch for the decision and groups that doubled; 1.52 for as many plain
+// rounds of three launches).
 // The vertex passes of a round take kStepPer vertices a thread (vertex base +
 // j * kBlock + t, coalesced), their loads issued first.  k_wpr_count: FP64 block
 // partials of sum |y|, and with a candidate extrapolation (cnt->ex.cand > 0) of the
@@ -155,10 +158,11 @@ constexpr int kStepPer = 4;
 
 template <class T>
 __global__ void __launch_bounds__(kBlock) k_wpr_count(uint32_t n, const T* __restrict__ x, const T* __restrict__ y,
-                                                      double* __restrict__ partial, const Counters* cnt) {
+                                                      double* __restrict__ partial, const Counters* cnt,
+                                                      const Extrap* __restrict__ ex) {
   __shared__ double s_p[2][kBlock / 64];
   if (cnt->done) return;
-  const double cand = cnt->ex.cand;
+  const double cand = ex->cand;
   const uint32_t base = blockIdx.x * (kBlock * kStepPer);
   T xo[kStepPer], xn[kStepPer];
 #pragma unroll
@@ -191,20 +195,22 @@ __global__ void __launch_bounds__(kBlock) k_wpr_count(uint32_t n, const T* __res
 }
 
 template <class T>
-__global__ void __launch_bounds__(kBlock) k_wpr_step(uint32_t n, T* __restrict__ x, T* __restrict__ y,
-                                                     T* __restrict__ sum, float* __restrict__ comp,
-                                                     const Counters* cnt, const uint32_t* __restrict__ pos,
-                                                     T* __restrict__ xc) {
-  if (cnt->done) return;
-  const double beta = cnt->ex.beta;
+__device__ __forceinline__ void wpr_step_load(uint32_t n, const T* __restrict__ x, const T* __restrict__ y,
+                                              T (&xo)[kStepPer], T (&xn)[kStepPer]) {
   const uint32_t base = blockIdx.x * (kBlock * kStepPer);
-  T xo[kStepPer], xn[kStepPer];
 #pragma unroll
   for (int j = 0; j < kStepPer; ++j) {
     const uint32_t v = base + j * kBlock + threadIdx.x;
     xo[j] = v < n ? x[v] : T(0);
     xn[j] = v < n ? y[v] : T(0);
   }
+}
+
+template <class T>
+__device__ __forceinline__ void wpr_step(uint32_t n, T* __restrict__ x, T* __restrict__ y, T* __restrict__ sum,
+                                         float* __restrict__ comp, double beta, const uint32_t* __restrict__ pos,
+                                         T* __restrict__ xc, const T (&xo)[kStepPer], T (&xn)[kStepPer]) {
+  const uint32_t base = blockIdx.x * (kBlock * kStepPer);
 #pragma unroll
   for (int j = 0; j < kStepPer; ++j) {
     const uint32_t v = base + j * kBlock + threadIdx.x;
@@ -220,6 +226,17 @@ __global__ void __launch_bounds__(kBlock) k_wpr_step(uint32_t n, T* __restrict__
       if (pos && pos[v] != INF32) xc[pos[v]] = xn[j];  // the next round gathers the compact copy
     }
   }
+}
+
+template <class T>
+__global__ void __launch_bounds__(kBlock) k_wpr_step(uint32_t n, T* __restrict__ x, T* __restrict__ y,
+                                                     T* __restrict__ sum, float* __restrict__ comp,
+                                                     const Counters* cnt, const uint32_t* __restrict__ pos,
+                                                     T* __restrict__ xc) {
+  if (cnt->done) return;
+  T xo[kStepPer], xn[kStepPer];
+  wpr_step_load<T>(n, x, y, xo, xn);
+  wpr_step<T>(n, x, y, sum, comp, cnt->ex.beta, pos, xc, xo, xn);
 }
 
 // l1: sum |seed|; the series stops at tol (relative: times l1).
@@ -240,6 +257,50 @@ __global__ void __launch_bounds__(1024) k_wpr_decide(const double* __restrict__ 
   cnt->edges += edges_per_round;
   if (s1 != s1 || s1 > 1e300) cnt->aux[0] = 1;
   if (!(r >= tol) || (long long)cnt->rounds >= (long long)max_rounds || cnt->aux[0]) cnt->done = 1;
+}
+
+// Decision and step of a round (its number from 0), gridDim.x <= kBlock: the same sums in
+// every workgroup, so the same decision.  The state it comes from is left alone
+// (ex2[round & 1]); the first workgroup writes the next one's and the counters.  One that
+// begins after the first has stopped the series finds `done` and would have stopped too.
+template <class T>
+__global__ void __launch_bounds__(kBlock) k_wpr_turn(uint32_t n, T* __restrict__ x, T* __restrict__ y,
+                                                     T* __restrict__ sum, float* __restrict__ comp, Counters* cnt,
+                                                     const uint32_t* __restrict__ pos, T* __restrict__ xc,
+                                                     const double* __restrict__ partial,
+                                                     const double* __restrict__ l1, double tol_abs, int relative,
+                                                     int round, int max_rounds, unsigned long long edges_per_round) {
+  __shared__ double s[kBlock / 64][2];
+  __shared__ double s_beta;
+  __shared__ int s_done, s_stop;
+  // everything that the decision and the step read, before either waits for it
+  T xo[kStepPer], xn[kStepPer];
+  wpr_step_load<T>(n, x, y, xo, xn);
+  Extrap ex = cnt->ex2[round & 1];
+  if (threadIdx.x == 0)  // one read for the workgroup: `done` may change meanwhile
+    s_done = __hip_atomic_load(&cnt->done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
+  sum_parts<2, 0u, kBlock>(partial, gridDim.x, s);  // waits for the workgroup
+  if (s_done) return;
+  if (threadIdx.x == 0) {
+    const double tol = relative ? tol_abs * *l1 : tol_abs;
+    const double s1 = s[0][0];
+    const double r = extrap_decide(ex, s1, s[0][1], tol);
+    const bool failed = s1 != s1 || s1 > 1e300;
+    s_beta = ex.beta;
+    s_stop = !(r >= tol) || round + 1 >= max_rounds || failed;
+    if (blockIdx.x == 0) {
+      cnt->ex2[~round & 1] = ex;
+      cnt->ex = ex;
+      cnt->dpad[0] = tol;
+      cnt->residual = r;
+      cnt->rounds = round + 1;
+      cnt->edges += edges_per_round;
+      if (failed) cnt->aux[0] = 1;
+      if (s_stop) __hip_atomic_store(&cnt->done, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+  }
+  __syncthreads();
+  if (!s_stop) wpr_step<T>(n, x, y, sum, comp, s_beta, pos, xc, xo, xn);
 }
 
 // x = scale * seed, y = sum = 0; block partials of sum |x|
@@ -286,7 +347,7 @@ __global__ void __launch_bounds__(1024) k_wpr_start(const double* __restrict__ p
   sum_parts<1, 0u>(partial, nparts, s);
   if (threadIdx.x == 0) {
     *l1 = s[0][0];
-    cnt->ex.last = s[0][0];
+    cnt->ex.last = cnt->ex2[0].last = s[0][0];
   }
 }
 
@@ -864,11 +925,18 @@ static void wpr_series(suminc_ctx* c, int& hint, const SeriesBufs<T>& B, const R
   // extrapolated series take 9-20 rounds, others up to hundreds, loose tolerances one or
   // two; a look at the counters costs about as much as three empty rounds
   int group = hint, enqueued = 0;
+  const bool turn = gs <= (unsigned)kBlock;
   while (true) {
     for (int i = 0; i < group; ++i, ++enqueued) {
       if (binned) bin_layout_spmv<T, true>(c, *L, pos ? xc : B.x, B.y, cnt, 2);
       else spmv<T>(c, R, a, pos ? xc : B.x, B.y, cnt);
-      k_wpr_count<T><<<gs, kBlock, 0, c->stream>>>(n, B.x, B.y, B.partial, cnt);
+      k_wpr_count<T><<<gs, kBlock, 0, c->stream>>>(n, B.x, B.y, B.partial, cnt,
+                                                  turn ? &cnt->ex2[enqueued & 1] : &cnt->ex);
+      if (turn) {
+        k_wpr_turn<T><<<gs, kBlock, 0, c->stream>>>(n, B.x, B.y, B.sum, B.comp, cnt, pos, xc, B.partial, B.l1, tol_abs,
+                                                   relative, enqueued, max_rounds, c->m);
+        continue;
+      }
       k_wpr_decide<<<1, 1024, 0, c->stream>>>(B.partial, gs, cnt, B.l1, tol_abs, relative, max_rounds, c->m);
       k_wpr_step<T><<<gs, kBlock, 0, c->stream>>>(n, B.x, B.y, B.sum, B.comp, cnt, pos, xc);
     }

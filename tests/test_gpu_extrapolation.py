@@ -227,6 +227,49 @@ def test_weighted_series_and_adjoint(gpu, prec, name):
     assert np.abs(gw - gw_want).max() <= tol * max(np.abs(gw_want).max(), np.abs(lam).max() * (want[u] / s[u]).max())
 
 
+@pytest.mark.parametrize("n", [1024, 1025, 1 << 18, (1 << 18) + 1])
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+def test_weighted_series_around_one_partial_a_thread(gpu, prec, n):
+    """Up to 2^18 vertices the step's workgroups decide for themselves, beyond a launch of
+    its own does: the same series, also where the round cap ends it."""
+    rng = np.random.default_rng(n)
+    u, v = rng.integers(0, n, 3 * n), rng.integers(0, n, 3 * n)
+    key = np.unique(u * n + v)
+    u, v = key // n, key % n
+    u, v = u[u != v], v[u != v]
+    off = np.zeros(n + 1, np.uint64)
+    off[1:] = np.cumsum(np.bincount(u, minlength=n))
+    w = (1.0 - rng.random(len(u))).astype(np.float32)
+    s = np.bincount(u, weights=w.astype(float), minlength=n)
+    M = sp.csr_matrix((DAMPING * w.astype(float) / s[u], (v, u)), shape=(n, n))
+    p = rng.random(n).astype(np.float32) / n
+    c = rng.standard_normal(n).astype(np.float32)
+    T = 1e-11 if prec == "fp64" else 1e-7
+    pr = gpu.PR_FP64 if prec == "fp64" else gpu.PR_FP32_KAHAN
+    x = (1 - DAMPING) * p.astype(float)
+    with gpu.Context(pr_precision=pr, termcheck_threshold=T, max_rounds=2000) as ctx:
+        ctx.upload_csr(off, v.astype(np.uint32), w)
+        ctx.wpr_set_weights(w)
+        for _ in range(2):  # the second run's first group is what the first one took
+            r, st = ctx.wpr_forward(p)
+            gp, _, sb = ctx.wpr_backward(c)
+        assert 1 < st["rounds"] <= plain_rounds_all(M, x, T) + 1 and st["residual"] < T
+        assert 1 < sb["rounds"] <= plain_rounds_all(M.T.tocsr(), c.astype(float), T * np.abs(c).sum()) + 1
+        ctx.set_params(max_rounds=5)
+        with pytest.raises(gpu.SumincError) as e:
+            ctx.wpr_forward(p)
+        assert e.value.code == gpu.E_NOT_CONVERGED
+        ctx.set_params(max_rounds=2000)
+        again, st2 = ctx.wpr_forward(p)
+    assert st2["rounds"] == st["rounds"]
+    want = series_limit(M, x)
+    tol = 1e-6 if prec == "fp64" else 1e-5  # rank and gradients come back as FP32
+    assert np.abs(r - want).sum() <= T / (1 - DAMPING) + tol
+    assert np.abs(again - want).sum() <= T / (1 - DAMPING) + tol
+    lam = series_limit(M.T.tocsr(), c.astype(float))
+    assert np.abs(gp - (1 - DAMPING) * lam).max() <= tol * np.abs(lam).max()
+
+
 def plain_rounds_all(M, x, T):
     k = 0
     while np.abs(x).sum() >= T:
