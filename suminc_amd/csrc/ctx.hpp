@@ -96,7 +96,6 @@ struct Extrap {
   double ratio;  // S2 / S1 of the previous round's candidate (0: none)
   double cand;   // the coefficient the next count evaluates (0: none)
   double beta;   // the coefficient the state's next vertex pass applies (0: none)
-  double steps;  // extrapolations taken
 };
 
 // Device-side counters block (one allocation, read back in one copy).

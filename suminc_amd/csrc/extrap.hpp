@@ -42,7 +42,6 @@ __device__ __forceinline__ double extrap_decide(Extrap& ex, double s1, double s2
   const double res = take ? s2 : s1;
   const double rho = !take && ex.last > 0.0 ? fmin(s1 / ex.last, kExtrapMaxRho) : 0.0;
   ex.beta = take ? ex.cand : 0.0;
-  ex.steps += take ? 1.0 : 0.0;
   ex.ratio = take ? 0.0 : q;
   ex.cand = rho / (1.0 - rho);
   ex.last = res;

@@ -123,7 +123,7 @@ def test_run_reaches_the_fixed_point(gpu, prec, name, seed):
 
 
 @pytest.mark.parametrize("name", ["ring", "communities", "uniform", "skewed"])
-@pytest.mark.parametrize("cap", [1, 2, 3, 5, 8, 9, 10, 11, 12, 14])
+@pytest.mark.parametrize("cap", [1, 2, 3, 5, 6, 8, 9, 10, 11, 12, 14])
 def test_round_cap_leaves_a_state_of_the_same_fixed_point(gpu, name, cap):
     n, u, v, off = graph(name)
     M = system(n, u, v)
@@ -137,10 +137,47 @@ def test_round_cap_leaves_a_state_of_the_same_fixed_point(gpu, name, cap):
         # the (untaken) rest of an inactive vertex stays in delta, so the state is exact
         assert np.abs(limit(M, r, d) - want).sum() < 1e-12
         assert np.abs(d).sum() <= (1 - DAMPING) * DAMPING ** st["rounds"] * (1 + 1e-9)
+        if (name, cap) in (("communities", 6), ("ring", 2), ("ring", 3)):
+            # the decision at the cap itself chose a step: far below as many plain rounds
+            assert np.abs(d).sum() < 0.1 * (1 - DAMPING) * DAMPING ** cap
         ctx.set_params(max_rounds=1000)
         ctx.pr_run()
         r, _ = ctx.pr_download()
     assert np.abs(r - want).sum() <= 1e-11 / (1 - DAMPING) + 1e-12
+
+
+@pytest.mark.parametrize("name,n", [("uniform", 3001), ("skewed", 4099), ("uniform", 1500)])
+@pytest.mark.parametrize("T", [1e-2, 1e-4, 1e-6, 1e-9, 1e-11])
+def test_runs_that_line_up_take_steps(gpu, name, n, T):
+    """On graphs whose series lines up the rounds fall well below plain ones', the last
+    decision takes a step too (the residual is below what the rounds alone reach), and the
+    state it leaves is exact.  1500 vertices: in one workgroup."""
+    n, u, v, off = graph(name) if n > 2048 else uniform(n)
+    M = system(n, u, v)
+    x = np.full(n, (1 - DAMPING) / n)
+    want = limit(M, np.zeros(n), x)
+    with gpu.Context(pr_precision=gpu.PR_FP64, termcheck_threshold=T, max_rounds=1000) as ctx:
+        ctx.upload_csr(off, v.astype(np.uint32))
+        ctx.pr_init()
+        st = ctx.pr_run()
+        r, d = ctx.pr_download()
+    plain = plain_rounds(M, x, T)
+    assert st["rounds"] <= 0.4 * plain + 1
+    k, y = 0, x
+    while k < st["rounds"]:
+        y, k = M @ y, k + 1
+    assert st["residual"] < T < 0.5 * np.abs(y).sum()
+    assert np.abs(limit(M, r, d) - want).sum() < 1e-12
+
+
+def uniform(n):
+    rng = np.random.default_rng(n)
+    key = np.unique(rng.integers(0, n, 6 * n) * n + rng.integers(0, n, 6 * n))
+    u, v = key // n, key % n
+    u, v = u[u != v], v[u != v]
+    off = np.zeros(n + 1, np.uint64)
+    off[1:] = np.cumsum(np.bincount(u, minlength=n))
+    return n, u, v, off
 
 
 def hubs(n=6007, hubs=300):
@@ -194,6 +231,59 @@ def test_sketch_run_reaches_the_fixed_point(gpu, prec, div):
                 assert e.code == gpu.E_NOT_CONVERGED
             r, d = ctx.pr_download()
             assert np.abs(limit(M, r, d) - want).sum() <= 0.15 * tol
+
+
+def test_sketch_rounds_take_steps_when_they_pull(gpu):
+    """Pulling sketch rounds that line up extrapolate (fewer rounds than pushing ones, which
+    do not), up to the decision that ends the phase, and every threshold leaves an exact
+    state: the entries', the exits' and the Singles' share of the last step."""
+    n, u, v, off = hubs()
+    M = system(n, u, v)
+    x = np.full(n, (1 - DAMPING) / n)
+    want = limit(M, np.zeros(n), x)
+    rounds = {}
+    for div in (1_000_000, 0):
+        with gpu.Context(pr_precision=gpu.PR_FP64, max_rounds=1000, pull_threshold_div=div) as ctx:
+            ctx.upload_csr(off, v.astype(np.uint32))
+            ctx.cluster_leaves(1024, 2)
+            for T in (1e-2, 1e-3, 1e-4, 1e-5, 1e-6, 1e-7, 1e-8):
+                ctx.set_params(termcheck_threshold=T)
+                ctx.sum_build(2, 1024, 1.0)
+                ctx.pr_upload(np.zeros(n), x)
+                rounds[div, T] = ctx.sum_pr_run()["sketch_rounds"]
+                r, d = ctx.pr_download()
+                assert np.abs(limit(M, r, d) - want).sum() < 1e-12
+                assert np.abs(d).sum() < T
+    for T in (1e-2, 1e-3, 1e-4, 1e-5, 1e-6, 1e-7, 1e-8):
+        assert rounds[1_000_000, T] <= 0.65 * rounds[0, T]
+
+
+@pytest.mark.parametrize("T", [1e-3, 1e-6, 1e-9])
+@pytest.mark.parametrize("big", [False, True], ids=["one_turn", "decide"])
+def test_weighted_series_that_line_up_take_steps(gpu, T, big):
+    """Rounds well below plain ones', and what the series leaves out is its residual's
+    share, which holds only if the step that ended it is in the result (2^18 + 1 vertices:
+    decided by a launch of its own)."""
+    n, u, v, off = uniform((1 << 18) + 1 if big else 3001)
+    w = (1.0 - np.random.default_rng(1).random(len(u))).astype(np.float32)
+    s = np.bincount(u, weights=w.astype(float), minlength=n)
+    M = sp.csr_matrix((DAMPING * w.astype(float) / s[u], (v, u)), shape=(n, n))
+    p = np.full(n, 1.0 / n, np.float32)
+    c = np.random.default_rng(2).random(n).astype(np.float32) + 0.5
+    x = (1 - DAMPING) * p.astype(float)
+    with gpu.Context(pr_precision=gpu.PR_FP64, termcheck_threshold=T, max_rounds=1000) as ctx:
+        ctx.upload_csr(off, v.astype(np.uint32), w)
+        ctx.wpr_set_weights(w)
+        _, st = ctx.wpr_forward(p)
+        r, _ = ctx.wpr_download()
+        _, _, sb = ctx.wpr_backward(c)
+        _, lam = ctx.wpr_download(adjoint=True)
+    assert st["rounds"] <= 0.5 * plain_rounds_all(M, x, T) + 1
+    assert sb["rounds"] <= 0.5 * plain_rounds_all(M.T.tocsr(), c.astype(float), T * np.abs(c).sum()) + 1
+    left = DAMPING / (1 - DAMPING)
+    assert np.abs(r - series_limit(M, x)).sum() <= left * st["residual"] * (1 + 1e-6) + 1e-12
+    # (d W contracts the maximum norm; on this graph the 1-norm grows by 2 at most)
+    assert np.abs(lam - series_limit(M.T.tocsr(), c.astype(float))).sum() <= 2 * left * sb["residual"] + 1e-9
 
 
 @pytest.mark.parametrize("name", ["ring", "path", "grid", "communities", "uniform", "skewed"])
