@@ -18,9 +18,17 @@
 // S2 is known to be the smaller: when it ends the run (S2 < T), or when S2 < S1 / 2 and
 // waiting another round no longer pays (S2 / S1 fell by less than kExtrapStall: as
 // the steps' polynomials commute, an extrapolation is worth the more the better rho is
-// known).  M does not grow the 1-norm, so sum |delta| after t rounds is never above
-// what t plain rounds guarantee, and a series that never lines up (an isolated cycle, a
-// path, signed mass on a regular grid) runs its plain rounds.
+// known).  A series that never lines up (an isolated cycle, a path, signed mass on a
+// regular grid) runs its plain rounds.
+//
+// What bounds the rounds: where M contracts the 1-norm by d (all forms but the adjoint's),
+// sum |delta| after t rounds is at most d^t of the first, steps or not, so a run ends by
+// the round at which that bound passes T.  A plain run may beat the bound by more than one
+// with steps does, from a single seed or where mass leaks through layers.  The adjoint's
+// transposed M contracts the maximum norm instead; its steps still halve the 1-norm each,
+// but there is no such bound.  Over some thousands of small random graphs (bipartite,
+// layered, cliques, stars, skewed, rings) the most was three rounds more than plain (45 ->
+// 48), two in the adjoint (32 -> 34), and none did not end.
 #pragma once
 #include "ctx.hpp"
 #include "device.hpp"

@@ -1,5 +1,6 @@
 """Extrapolated delta series: wherever a run stops, rank and delta are a state of the
-same fixed point, r + (I - M)^-1 delta, and no graph takes more rounds than plain ones.
+same fixed point, r + (I - M)^-1 delta, and these graphs take no more rounds than plain
+ones (one more where sums may cross T a round later).
 
 Graphs: ones whose series lines up with one eigenvector (R-MAT, uniform, communities),
 ones that are eigenvectors from the start (ring, pairs) and ones that never line up
