@@ -858,10 +858,11 @@ __global__ void k_insert_relax(const uint32_t* grow, const uint32_t* gcol, const
     v = gcol[g];
     uint32_t du = (uint32_t)(dp[u] >> 32);
     unsigned long long nd = trav_extend(app, du, unit ? 1u : gw[g]);
+    const unsigned long long seen = dp[v];
     // SSWP: strictly better values only (trav_commit)
-    if (du != INF32 && nd < INF32 && (app != SUMINC_APP_SSWP || nd < (dp[v] >> 32))) {
+    if (du != INF32 && nd < INF32 && (app != SUMINC_APP_SSWP || nd < (seen >> 32))) {
       unsigned long long cand = (nd << 32) | u;
-      unsigned long long old = trav_commit(app, &dp[v], cand);
+      unsigned long long old = trav_commit(app, &dp[v], cand, seen);
       if ((old >> 32) > nd) {
         uint32_t bit = 1u << (v & 31);
         add = !(atomicOr(&bits0[v >> 5], bit) & bit);

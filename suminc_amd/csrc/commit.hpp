@@ -23,13 +23,15 @@
 
 namespace suminc {
 
-// Cell: load(), fetch_min(x) and compare_exchange(expected, x), each returning the word
-// that was there.  Returns the word that cand met: the value (high half) fell if it is
-// above cand's.
+// Cell: fetch_min(x) and compare_exchange(expected, x), each returning the word that was
+// there.  seen: the word as the caller last read it, however long ago.  Returns the word
+// that cand met (SSWP: or the last one seen, when that already rules cand out): the value
+// (high half) fell if it is above cand's.
 template <class Cell>
-SUMINC_HOST_DEVICE unsigned long long trav_commit(int app, Cell cell, unsigned long long cand) {
+SUMINC_HOST_DEVICE unsigned long long trav_commit(int app, Cell cell, unsigned long long cand,
+                                                  unsigned long long seen) {
   if (app != SUMINC_APP_SSWP) return cell.fetch_min(cand);
-  unsigned long long now = cell.load();
+  unsigned long long now = seen;
   while ((cand >> 32) < (now >> 32)) {  // a failed exchange finds a smaller word: it ends
     const unsigned long long was = cell.compare_exchange(now, cand);
     if (was == now) break;

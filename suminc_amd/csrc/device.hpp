@@ -138,14 +138,14 @@ __device__ __forceinline__ unsigned long long trav_extend(int app, uint32_t word
 // trav_commit on a word in device memory.
 struct DpCell {
   unsigned long long* p;
-  __device__ unsigned long long load() const { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
   __device__ unsigned long long fetch_min(unsigned long long x) const { return atomicMin(p, x); }
   __device__ unsigned long long compare_exchange(unsigned long long expected, unsigned long long x) const {
     return atomicCAS(p, expected, x);
   }
 };
-__device__ __forceinline__ unsigned long long trav_commit(int app, unsigned long long* p, unsigned long long cand) {
-  return trav_commit(app, DpCell{p}, cand);
+__device__ __forceinline__ unsigned long long trav_commit(int app, unsigned long long* p, unsigned long long cand,
+                                                          unsigned long long seen) {
+  return trav_commit(app, DpCell{p}, cand, seen);
 }
 
 }  // namespace suminc

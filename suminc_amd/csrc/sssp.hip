@@ -61,8 +61,9 @@ __device__ __forceinline__ void sssp_relax(const SsspArgs& a, int nxt, uint32_t 
     // words only decrease while the rounds run: a candidate no smaller than a
     // plain (possibly stale) read cannot win, so it skips the atomic.  SSWP takes
     // strictly better values only (trav_commit)
-    if (a.app == SUMINC_APP_SSWP ? nd < (a.dp[v] >> 32) : cand < a.dp[v]) {
-      unsigned long long old = trav_commit(a.app, &a.dp[v], cand);
+    const unsigned long long seen = a.dp[v];
+    if (a.app == SUMINC_APP_SSWP ? nd < (seen >> 32) : cand < seen) {
+      unsigned long long old = trav_commit(a.app, &a.dp[v], cand, seen);
       add = (old >> 32) > nd;
     }
   }
@@ -216,7 +217,7 @@ __global__ void __launch_bounds__(kBlock) k_sssp_pull(SsspArgs a, SsspPull p) {
       if (nd >= INF32) continue;
       const unsigned long long cand = nd << 32 | u, was = a.dp[lo];
       if (!sssp_better(a.app, cand, was, (uint32_t)(was >> 32))) continue;
-      if ((trav_commit(a.app, &a.dp[lo], cand) >> 32) > nd) sssp_mark(a.bits[nxt], lo);
+      if ((trav_commit(a.app, &a.dp[lo], cand, was) >> 32) > nd) sssp_mark(a.bits[nxt], lo);
     }
   } else {
 #pragma unroll
@@ -300,11 +301,13 @@ __global__ void __launch_bounds__(kBlock) k_sssp_pull(SsspArgs a, SsspPull p) {
       const uint32_t i = j * kBlock + threadIdx.x, v = s_id[i];
       if (v == INF32) continue;
       const unsigned long long best = s_min[i];
-      if (best == 0ull || best >= a.dp[v]) continue;
+      if (best == 0ull) continue;
+      const unsigned long long seen = a.dp[v];
+      if (best >= seen) continue;
       if (p.ioff[v] >= e0 && p.ioff[v + 1] <= e0 + ne) {
         a.dp[v] = best;
         if ((uint32_t)(best >> 32) < s_old[i]) sssp_mark(a.bits[nxt], v);
-      } else if ((trav_commit(a.app, &a.dp[v], best) >> 32) > (best >> 32)) {
+      } else if ((trav_commit(a.app, &a.dp[v], best, seen) >> 32) > (best >> 32)) {
         sssp_mark(a.bits[nxt], v);
       }
     }

@@ -16,6 +16,7 @@ struct Shared {
   u64 now;
   std::vector<u64> others;
   size_t at = 0;
+  u64 replaced = ~0ull;  // the word that trav_commit wrote over
   void interfere() {
     if (at < others.size() && others[at] != ~0ull) {
       const u64 x = others[at];
@@ -26,20 +27,22 @@ struct Shared {
 };
 struct Cell {
   Shared* s;
-  u64 load() const {
-    s->interfere();
-    return s->now;
-  }
   u64 fetch_min(u64 x) const {
     s->interfere();
     const u64 was = s->now;
-    if (x < was) s->now = x;
+    if (x < was) {
+      s->replaced = was;
+      s->now = x;
+    }
     return was;
   }
   u64 compare_exchange(u64 expected, u64 x) const {
     s->interfere();
     const u64 was = s->now;
-    if (was == expected) s->now = x;
+    if (was == expected) {
+      s->replaced = was;
+      s->now = x;
+    }
     return was;
   }
 };
@@ -53,7 +56,8 @@ struct Cell {
   } while (0)
 
 int main() {
-  // every word, candidate and pair of interfering words over small values and parents
+  // every word as it was read, interfering words since and candidate, over small values
+  // and parents
   std::vector<u64> words;
   for (u64 v = 0; v < 4; ++v)
     for (u64 p = 0; p < 3; ++p) words.push_back(word(v, p));
@@ -65,11 +69,11 @@ int main() {
         for (u64 b : others)
           for (u64 cand : words) {
             Shared s{app, first, {a, b}};
-            const u64 met = trav_commit(app, Cell{&s}, cand);
+            const u64 met = trav_commit(app, Cell{&s}, cand, first);
             if (app == SUMINC_APP_SSWP) {
-              const bool took = (cand >> 32) < (met >> 32);
-              if (took) CHECK(s.now == cand || (s.now >> 32) < (cand >> 32));
-              else CHECK(s.now == met);  // a tie leaves the word as it was met, its parent too
+              // written over a strictly worse value only, and reported as such
+              CHECK((s.replaced != ~0ull) == ((cand >> 32) < (met >> 32)));
+              if (s.replaced != ~0ull) CHECK(s.replaced == met && s.now == cand);
             } else {
               CHECK(s.now == (cand < met ? cand : met));
             }
@@ -82,11 +86,11 @@ int main() {
     const u64 W = 5, old = 9;
     Shared v{SUMINC_APP_SSWP, word(old, 7), {}}, u2{SUMINC_APP_SSWP, word(old, 7), {}};
     const u64 b_old = v.now >> 32;
-    trav_commit(SUMINC_APP_SSWP, Cell{&v}, word(W, 2));
-    trav_commit(SUMINC_APP_SSWP, Cell{&u2}, word(v.now >> 32, 0));
+    trav_commit(SUMINC_APP_SSWP, Cell{&v}, word(W, 2), v.now);
+    trav_commit(SUMINC_APP_SSWP, Cell{&u2}, word(v.now >> 32, 0), u2.now);
     const u64 best = word(u2.now >> 32, 1);
     CHECK((best >> 32) < b_old);  // B's own test lets it pass
-    trav_commit(SUMINC_APP_SSWP, Cell{&v}, best);
+    trav_commit(SUMINC_APP_SSWP, Cell{&v}, best, word(old, 7));
     CHECK((u2.now & 0xFFFFFFFFu) == 0);
     CHECK((v.now & 0xFFFFFFFFu) == 2);
   }
