@@ -20,7 +20,8 @@ using namespace suminc;
 
 // One read-back of `count` chunks of up to 64 bytes; 0: all there, 1: wrong, 2: bad_alloc.
 static int run(size_t count, bool threaded, long fail) {
-  std::vector<unsigned char> slots(kSlots * kChunkBytes), out(count * 64, 0);
+  static std::vector<unsigned char> slots(kSlots * kChunkBytes);
+  std::vector<unsigned char> out(count * 64, 0);
   std::vector<Chunk> chunks;
   for (size_t i = 0; i < count; ++i) chunks.push_back({0, i, 1, &out[i * 64], 1 + i % 64});
   try {
